@@ -323,7 +323,7 @@ extern "C" int ga_alm2map_spin_f64(const ga_plan *p, int32_t spin, const double 
   GA_REQUIRE(ws_bytes >= ring_bytes(p, 2, 8), GA_ERR_WORKSPACE, "workspace %zu < %zu bytes",
              ws_bytes, ring_bytes(p, 2, 8));
   hipStream_t s = (hipStream_t)stream;
-  int rc = launch_spin_synth_f64(p, spin, 1, E, B, (double *)ws, s);
+  int rc = launch_spin_synth_f64(p, spin, E, B, (double *)ws, s);
   if (rc) return rc;
   return launch_ring_synth_f64(p, 2, 2, (const double *)ws, maps, nullptr, s);
 }

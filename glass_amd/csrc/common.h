@@ -91,6 +91,14 @@ __host__ __device__ inline int ring_group(int nshell) { return nshell >= 8 ? 8 :
 // log2 of the real columns (2 G) per group
 __host__ __device__ inline int ring_group_cshift(int nshell) { return nshell >= 8 ? 4 : 3; }
 
+// Block order of the FP64 Legendre stages: block b runs on XCD b % 8, which
+// takes the runs of eight consecutive m starting at 8 x, 8 x + 64, ... (the
+// 16-byte ring coefficients of eight m share a 128-byte line, written and
+// read through one XCD's L2), small m (the long sums) first, the nrg ring
+// groups of one m back to back.
+__host__ __device__ inline unsigned m_run8_blocks(int lmax, int nrg) {
+  return unsigned(64 * ((lmax + 64) / 64) * nrg);
+}
 // l rows per slab of the FP16-split MFMA Legendre stage (K = 16 per parity)
 constexpr int kSlab = 32;
 __host__ __device__ inline int64_t nslab_of(int64_t lmax, int64_t m) { return (lmax - m + kSlab) / kSlab; }

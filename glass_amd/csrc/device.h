@@ -119,6 +119,29 @@ __device__ __forceinline__ void to_scaled(double mant, long long E, double &p, i
   p = ldexp(mant, rem);
 }
 
+// The scaled form of the FP64 stages: value = p 2^(600 k), k <= 0, where a
+// scaled value (k < 0) is held below 2^-300.  Such a p stands for a number
+// below 2^-900 of its own magnitude, so a kernel may use it as if it were the
+// value: the error it makes is below 2^-200 of the operand it multiplies (a
+// chunk of 16 recurrence steps grows a value by less than 2^100), and no
+// step needs a test.  rescale_low is called once per chunk and moves a value
+// that has passed 2^-300 up one scale.
+constexpr int kLowBits = 300;
+
+__device__ __forceinline__ void to_scaled_low(double mant, long long E, double &p, int &k) {
+  const long long negE = -E;
+  k = negE < kLowBits + kScaleBits ? 0 : -int((negE - kLowBits) / kScaleBits);
+  p = ldexp(mant, int(E - (long long)kScaleBits * k));
+}
+
+__device__ __forceinline__ void rescale_low(double &p0, double &p1, int &k) {
+  if (k < 0 && fabs(p1) > 0x1p-300) {
+    p1 *= 0x1p-600;
+    p0 *= 0x1p-600;
+    ++k;
+  }
+}
+
 // ---- Philox4x32-10 (Salmon, Moraes, Dror, Shaw 2011), counter-based
 struct u32x4 {
   uint32_t v[4];
@@ -141,6 +164,15 @@ __device__ __forceinline__ u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1
 // a double in [0, 1) with 53 random bits from two words (27 + 26 bits)
 __device__ __forceinline__ double uniform53(uint32_t a, uint32_t b) {
   return (double(a >> 5) * 67108864.0 + double(b >> 6)) * 0x1p-53;
+}
+
+// (m, ring group) of this block of a grid of m_run8_blocks (see common.h)
+__device__ __forceinline__ bool decode_m_run8(int lmax, int nrg, int &m, int &rg) {
+  const int b = blockIdx.x, xcd = b & 7, kq = b >> 3;
+  const int mq = kq / nrg;
+  rg = kq - mq * nrg;
+  m = 64 * (mq >> 3) + 8 * xcd + (mq & 7);
+  return m <= lmax;
 }
 
 // full 64-bit lane masks

@@ -87,8 +87,9 @@ int launch_legendre_anal_f16(const ga_plan *p, int S, const float *F, float *par
 
 // Spin synthesis Legendre stage: (E, B) [idx][S] -> ring buffer [ring][m][2S],
 // column 2s = Q_s, 2s + 1 = U_s
-int launch_spin_synth_f64(const ga_plan *p, int spin, int S, const double *E, const double *B,
-                          double *Fo, hipStream_t s);
+// (FP64: one pair of maps, S = 1)
+int launch_spin_synth_f64(const ga_plan *p, int spin, const double *E, const double *B, double *Fo,
+                          hipStream_t s);
 int launch_spin_synth_f32(const ga_plan *p, int spin, int S, const float *E, const float *B,
                           float *Fo, hipStream_t s);
 // Spin synthesis Legendre stage on split-FP16 MFMA: E (and B, may be NULL for

@@ -9,9 +9,9 @@
 // its own partial [wave][idx][s]; a second kernel sums the waves in a fixed
 // order, so the result does not depend on scheduling.
 //
-// The spin-s synthesis (alm2map_spin) stage lives here too: one lane per
-// (m, ring pair) running the +s and -s Wigner-d recurrences, with the E/B alm
-// read as wave-uniform values.
+// The FP32 VALU form of the spin-s synthesis (alm2map_spin) stage lives here
+// too: one lane per (m, ring pair) running the +s and -s Wigner-d recurrences,
+// with the E/B alm read as wave-uniform values.
 #include "common.h"
 #include "device.h"
 #include "kernels.h"
@@ -280,10 +280,6 @@ static int launch_spin(const ga_plan *p, int spin, int S, const T *E, const T *B
   return GA_OK;
 }
 
-int launch_spin_synth_f64(const ga_plan *p, int spin, int S, const double *E, const double *B,
-                          double *Fo, hipStream_t s) {
-  return launch_spin<double>(p, spin, S, E, B, Fo, s);
-}
 int launch_spin_synth_f32(const ga_plan *p, int spin, int S, const float *E, const float *B,
                           float *Fo, hipStream_t s) {
   return launch_spin<float>(p, spin, S, E, B, Fo, s);

@@ -1,0 +1,44 @@
+"""The FP64 Legendre stages where their loops change shape: band limits around
+a whole number of chunks of rows, ring-pair counts around whole waves, fewer
+rows than the spin, and m so large that the polar rings' values start
+thousands of binary orders below one.
+
+Tolerance: one FP64 recurrence step perturbs a value by a few ulp, and the
+perturbations of lmax steps add, so max |error| / RMS of the oracle's result
+stays below 64 (lmax + 1) 2^-52.
+"""
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+from glass_amd import healpix as hp  # noqa: E402
+
+
+def rand_alm(lmax, rng):
+    n = O.nalm(lmax)
+    return rng.standard_normal(n) + 1j * rng.standard_normal(n)
+
+
+def bound(lmax):
+    return 64 * (lmax + 1) * 2.0**-52
+
+
+@pytest.mark.parametrize("spin", [1, 2])
+@pytest.mark.parametrize("nside,lmax", [(1, 1), (1, 2), (3, 6), (5, 7), (16, 8), (31, 15), (33, 17),
+                                        (96, 64), (130, 41), (40, 600)])
+def test_spin_synthesis_edges(spin, nside, lmax):
+    print(f"spin={spin} nside={nside} lmax={lmax}", flush=True)
+    rng = np.random.default_rng(1000 * nside + 10 * lmax + spin)
+    E, B = rand_alm(lmax, rng), rand_alm(lmax, rng)
+    rq, ru = O.alm2map_spin([E, B], nside, spin, lmax, nthreads=4)
+    q, u = hp.alm2map_spin([E, B], nside, spin, lmax)
+    scale = np.sqrt(np.mean(rq**2 + ru**2))
+    if scale == 0:  # lmax < spin: nothing to synthesise
+        assert not q.any() and not u.any()
+        return
+    assert np.max(np.abs(q - rq)) / scale < bound(lmax)
+    assert np.max(np.abs(u - ru)) / scale < bound(lmax)
