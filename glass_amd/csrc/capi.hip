@@ -269,8 +269,8 @@ static int map2alm_impl(const ga_plan *p, int S, const T *map, T *alm, int niter
     if (sizeof(T) == 8) {
       rc = launch_ring_anal_f64(p, S, (const double *)src, (double *)F, s);
       if (rc) return rc;
-      rc = launch_legendre_anal_f64(p, S, (const double *)F, (double *)alm, (double *)partial,
-                                    it > 0, s);
+      rc = launch_legendre_anal_f64(p, (const double *)F, (double *)alm, (double *)partial, it > 0,
+                                    s);
     } else {
       rc = launch_ring_anal_f32(p, S, (const float *)src, (float *)F, s);
       if (rc) return rc;

@@ -52,11 +52,12 @@ __device__ __forceinline__ cplx<float> expi_frac(int64_t q, int64_t d, float) {
 // sin^m is formed by binary powering with exact exponent bookkeeping.
 constexpr int kScaleBits = 600;
 
-__device__ __forceinline__ void legendre_seed(double cm, double sth, int m, double &p,
-                                              int &k) {
+// sin^m(theta) = rm 2^E (E <= 0), with exact exponent bookkeeping
+__device__ __forceinline__ void sin_power(double sth, int m, double &rm, long long &E) {
   int es;
   double b = frexp(sth, &es);  // sth = b 2^es, b in [0.5, 1)
-  double rm = 1.0, bm = b;
+  double bm = b;
+  rm = 1.0;
   int er = 0, eb = 0;
   int mm = m;
   while (mm) {
@@ -72,7 +73,14 @@ __device__ __forceinline__ void legendre_seed(double cm, double sth, int m, doub
       eb = 2 * eb + t;
     }
   }
-  const long long E = (long long)er + (long long)m * (long long)es;  // <= 0
+  E = (long long)er + (long long)m * (long long)es;  // <= 0
+}
+
+__device__ __forceinline__ void legendre_seed(double cm, double sth, int m, double &p,
+                                              int &k) {
+  double rm;
+  long long E;
+  sin_power(sth, m, rm, E);
   const long long negE = -E;
   k = -int(negE / kScaleBits);
   const int rem = int(E + (long long)kScaleBits * (negE / kScaleBits));  // in (-600, 0]
@@ -134,12 +142,21 @@ __device__ __forceinline__ void to_scaled_low(double mant, long long E, double &
   p = ldexp(mant, int(E - (long long)kScaleBits * k));
 }
 
+// the seed lambda_mm in that form
+__device__ __forceinline__ void legendre_seed_low(double cm, double sth, int m, double &p,
+                                                  int &k) {
+  double rm;
+  long long E;
+  sin_power(sth, m, rm, E);
+  to_scaled_low(cm * rm, E, p, k);
+}
+
 __device__ __forceinline__ void rescale_low(double &p0, double &p1, int &k) {
-  if (k < 0 && fabs(p1) > 0x1p-300) {
-    p1 *= 0x1p-600;
-    p0 *= 0x1p-600;
-    ++k;
-  }
+  const bool up = k < 0 && fabs(p1) > 0x1p-300;
+  const double f = up ? 0x1p-600 : 1.0;
+  p1 *= f;
+  p0 *= f;
+  k += up;
 }
 
 // ---- Philox4x32-10 (Salmon, Moraes, Dror, Shaw 2011), counter-based

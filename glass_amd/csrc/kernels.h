@@ -76,8 +76,12 @@ int launch_ring_resid_f32(const ga_plan *p, int S, int G, const float *F, float 
 // Legendre stage of analysis: F [ring][m][S] -> alm [idx][S] (+= when accumulate)
 // partial: anal_partial_slots(p) * nalm * S complex scratch
 int anal_partial_slots(const ga_plan *p);
-int launch_legendre_anal_f64(const ga_plan *p, int S, const double *F, double *alm,
-                             double *partial, bool accumulate, hipStream_t s);
+// (FP64: one map, S = 1)
+int launch_legendre_anal_f64(const ga_plan *p, const double *F, double *alm, double *partial,
+                             bool accumulate, hipStream_t s);
+// alm (+)= the nw partial sums of n values each, added in order
+int launch_reduce_partials_f64(int64_t n, int nw, const double *partial, double *alm,
+                               bool accumulate, hipStream_t s);
 int launch_legendre_anal_f32(const ga_plan *p, int S, const float *F, float *alm, float *partial,
                              bool accumulate, hipStream_t s);
 // the split-FP16 MFMA form of the FP32 analysis contraction: F -> partial

@@ -1,4 +1,4 @@
-// Legendre stage of the analysis (map2alm), VALU version, FP64 and FP32.
+// Legendre stage of the analysis (map2alm), FP32 VALU version.
 //
 //   a_lm[s] = sum_rp lambda_lm(theta_rp) ( F_N[rp, m, s] + (-1)^(l+m) F_S[rp, m, s] )
 //
@@ -36,12 +36,6 @@ __device__ __forceinline__ float wave_sum_last(float v) {
   v = dpp_add<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
   return v;                    // lane 63: the wave's sum
 }
-__device__ __forceinline__ double wave_sum_last(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;  // every lane (the FP64 path keeps the exact butterfly order)
-}
-
 constexpr int kAnalRPL = 8;  // ring pairs per lane
 
 template <typename T, int SC>
@@ -234,35 +228,35 @@ __global__ __launch_bounds__(256) void spin_synth_kernel(
 int anal_partial_slots(const ga_plan *p) { return (p->npairs + 64 * kAnalRPL - 1) / (64 * kAnalRPL); }
 
 template <typename T>
-static int launch_anal(const ga_plan *p, int S, const T *F, T *alm, T *partial, bool accumulate,
-                       hipStream_t stream) {
-  const int nw = anal_partial_slots(p);
-  if (sizeof(T) == 4 && p->tune.anal_path != 1) {
-    int rc = launch_legendre_anal_f16(p, S, (const float *)F, (float *)partial, stream);
-    if (rc) return rc;
-  } else {
-    const int nblk_y = (nw + 3) / 4;
-    constexpr int SC = sizeof(T) == 8 ? 1 : 2;
-    dim3 grid(unsigned(p->lmax + 1), unsigned(nblk_y), unsigned((S + SC - 1) / SC));
-    hipLaunchKernelGGL((legendre_anal_kernel<T, SC>), grid, dim3(256), 0, stream, p->lmax,
-                       p->npairs, p->nrings, S, p->d_z, p->d_sth, p->d_ab, p->d_cm,
-                       (const cplx<T> *)F, (cplx<T> *)partial, p->nalm);
-    GA_LAUNCH_CHECK();
-  }
-  const int64_t n = p->nalm * S;
+static int launch_reduce(int64_t n, int nw, const T *partial, T *alm, bool accumulate,
+                         hipStream_t stream) {
   hipLaunchKernelGGL(reduce_partials_kernel<T>, dim3(unsigned((n + 255) / 256)), dim3(256), 0,
                      stream, n, nw, (const cplx<T> *)partial, (cplx<T> *)alm, accumulate ? 1 : 0);
   GA_LAUNCH_CHECK();
   return GA_OK;
 }
 
-int launch_legendre_anal_f64(const ga_plan *p, int S, const double *F, double *alm,
-                             double *partial, bool accumulate, hipStream_t s) {
-  return launch_anal<double>(p, S, F, alm, partial, accumulate, s);
+int launch_reduce_partials_f64(int64_t n, int nw, const double *partial, double *alm,
+                               bool accumulate, hipStream_t s) {
+  return launch_reduce(n, nw, partial, alm, accumulate, s);
 }
+
 int launch_legendre_anal_f32(const ga_plan *p, int S, const float *F, float *alm, float *partial,
-                             bool accumulate, hipStream_t s) {
-  return launch_anal<float>(p, S, F, alm, partial, accumulate, s);
+                             bool accumulate, hipStream_t stream) {
+  const int nw = anal_partial_slots(p);
+  if (p->tune.anal_path != 1) {
+    int rc = launch_legendre_anal_f16(p, S, F, partial, stream);
+    if (rc) return rc;
+  } else {
+    const int nblk_y = (nw + 3) / 4;
+    constexpr int SC = 2;
+    dim3 grid(unsigned(p->lmax + 1), unsigned(nblk_y), unsigned((S + SC - 1) / SC));
+    hipLaunchKernelGGL((legendre_anal_kernel<float, SC>), grid, dim3(256), 0, stream, p->lmax,
+                       p->npairs, p->nrings, S, p->d_z, p->d_sth, p->d_ab, p->d_cm,
+                       (const cplx<float> *)F, (cplx<float> *)partial, p->nalm);
+    GA_LAUNCH_CHECK();
+  }
+  return launch_reduce(p->nalm * S, nw, partial, alm, accumulate, stream);
 }
 
 template <typename T>

@@ -42,3 +42,18 @@ def test_spin_synthesis_edges(spin, nside, lmax):
         return
     assert np.max(np.abs(q - rq)) / scale < bound(lmax)
     assert np.max(np.abs(u - ru)) / scale < bound(lmax)
+
+
+# npairs = 2 nside: one wave (<= 64 pairs), two to four waves, two / four / eight
+# pairs per lane (from 257, 513, 1025 pairs), two workgroups for each m (2060)
+@pytest.mark.parametrize("nside,lmax,niter", [(1, 0, 0), (1, 4, 1), (32, 14, 0), (33, 15, 1),
+                                              (100, 16, 0), (128, 31, 0), (129, 33, 1),
+                                              (257, 47, 0), (513, 40, 0), (1030, 20, 1),
+                                              (40, 600, 0)])
+def test_analysis_edges(nside, lmax, niter):
+    print(f"analysis nside={nside} lmax={lmax} niter={niter}", flush=True)
+    rng = np.random.default_rng(nside + 7 * lmax)
+    f = rng.standard_normal(12 * nside * nside)
+    ref = O.map2alm(f, lmax, niter=niter, nthreads=8)
+    got = hp.map2alm(f, lmax=lmax, iter=niter)
+    assert np.max(np.abs(got - ref)) / np.sqrt(np.mean(np.abs(ref) ** 2)) < bound(lmax)
