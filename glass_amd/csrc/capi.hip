@@ -68,7 +68,11 @@ extern "C" int ga_alm2map_f64(const ga_plan *p, const double *alm, double *map, 
              "workspace %zu < %zu bytes", ws_bytes, ring_bytes(p, 1, 8));
   hipStream_t s = (hipStream_t)stream;
   double *F = (double *)ws;
-  int rc = launch_legendre_synth_f64(p, alm, F, s);
+  // the map is written by the ring stage alone: scratch of the Legendre stage,
+  // unless a caller keeps the alm in the same memory
+  const bool apart = alm + 2 * p->nalm <= map || map + p->npix <= alm;
+  int rc = launch_legendre_synth_f64(p, alm, F, apart ? map : nullptr,
+                                     apart ? size_t(p->npix) : 0, s);
   if (rc) return rc;
   return launch_ring_synth_f64(p, 1, 1, F, map, nullptr, s);
 }
@@ -236,7 +240,8 @@ static int map2alm_impl(const ga_plan *p, int S, const T *map, T *alm, int niter
       // map_tmp = map - S(alm)
       bool subtract = true;
       if (sizeof(T) == 8) {
-        rc = launch_legendre_synth_f64(p, (const double *)alm, (double *)F, s);
+        rc = launch_legendre_synth_f64(p, (const double *)alm, (double *)F, (double *)map_tmp,
+                                       size_t(p->npix), s);
         if (rc) return rc;
         rc = launch_ring_synth_f64(p, 1, 1, (const double *)F, (double *)map_tmp, nullptr, s);
       } else {

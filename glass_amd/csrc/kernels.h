@@ -5,8 +5,11 @@
 
 namespace ga {
 
-// Legendre stage, FP64 plain: alm (healpy order complex128) -> F [ring][m] complex128
-int launch_legendre_synth_f64(const ga_plan *p, const double *alm, double *F, hipStream_t s);
+// Legendre stage, FP64 plain: alm (healpy order complex128) -> F [ring][m] complex128.
+// scratch: memory the stage may overwrite (with room for the alm it runs the
+// faster form; NULL, 0 for none), neither alm nor F
+int launch_legendre_synth_f64(const ga_plan *p, const double *alm, double *F, double *scratch,
+                              size_t scratch_doubles, hipStream_t s);
 
 // Legendre stage, FP32 MFMA batched: alm [idx][S] complex64 -> F (grouped ring buffer)
 int launch_legendre_synth_mfma(const ga_plan *p, const ga_tuning &tu, int S, const float *alm,

@@ -1,13 +1,26 @@
 // Plain FP64 Legendre stage of the scalar synthesis (one map, no MFMA).
 //
-// One lane per (m, ring pair).  The lane runs the normalised associated-
-// Legendre recurrence in l for its ring's cos(theta) in FP64 (seed
-// lambda_mm = c_m sin^m theta carried with a 2^600-step scale index so it never
-// underflows), and accumulates the l-sums of a_lm lambda_lm split by the parity
-// of l - m, which gives the north ring and its south mirror at once:
+// A lane owns RPL ring pairs of one m and runs the associated-Legendre recurrence
+// in l for their cos(theta) in FP64, from the seed lambda_mm = c_m sin^m theta.  It
+// accumulates the l-sums of a_lm lambda_lm split by the parity of l - m (static in
+// the unrolled loop), which gives the north ring and its south mirror at once:
 //     F_m(theta)      = E + O,   F_m(pi - theta) = E - O,
 // because lambda_lm(-x) = (-1)^(l+m) lambda_lm(x).
-// This is the honest FP64 baseline the batched FP32-MFMA path is compared to.
+//
+// Coefficients and alm are wave-uniform: scalar loads, kRows rows at a time,
+// which serve all RPL pairs.  Values far below the range that matters are kept
+// scaled (to_scaled_low) and rescaled every 2 kRows rows, so no step has a test.
+// NORM runs the normalised form y_l = lambda_l / c_l, two operations a step
+// instead of three, against alm that a first pass has multiplied by c_l; the
+// plain form (a, a b) reads the alm as they are and saves that launch.
+//
+// Bound: FP64 issue, 4 (NORM) or 5 operations per (l, m, ring pair).  Measured at
+// nside 1024, lmax 2048: 705 us (one pair per lane, a test of the scale and
+// three operations in each step: 1377 us), of which the seeds take 80 us and
+// the stores 20.  Issuing each batch of scalar loads one turn ahead changed
+// nothing (716 against 711 us), four pairs per lane neither.
+#include <algorithm>
+
 #include "common.h"
 #include "device.h"
 #include "kernels.h"
@@ -16,105 +29,148 @@ namespace ga {
 
 namespace {
 
+constexpr int kRows = 8;           // rows per batch of scalar loads
+constexpr int64_t kManyWaves = 16384;  // see launch_legendre_synth_f64
+
+template <int RPL, bool NORM>
+struct synth_state {
+  double x[RPL], p0[RPL], p1[RPL];
+  double2 acc[2][RPL];  // by the parity of l - m
+  int k[RPL];
+
+  // one row: c = (gam, -) or (a, a b)
+  __device__ __forceinline__ void step(int par, double2 c, double2 a) {
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      const double y = fma(c.x * x[j], p1[j], NORM ? -p0[j] : -(c.y * p0[j]));
+      p0[j] = p1[j];
+      p1[j] = y;
+      acc[par][j].x = fma(y, a.x, acc[par][j].x);
+      acc[par][j].y = fma(y, a.y, acc[par][j].y);
+    }
+  }
+};
+
+template <bool NORM>
+__device__ __forceinline__ double2 row_coef(const double *__restrict__ t, int i) {
+  return NORM ? double2{t[i], 0.0} : reinterpret_cast<const double2 *>(t)[i];
+}
+
+template <int RPL, bool NORM>
 __global__ __launch_bounds__(256) void legendre_synth_f64_kernel(
-    int lmax, int npairs, int nrings, const double *__restrict__ z,
-    const double *__restrict__ sth, const double2 *__restrict__ ab,
+    int lmax, int npairs, int nrings, int nrg, const double *__restrict__ z,
+    const double *__restrict__ sth, const double *__restrict__ tab /* gam, or (a, a b) */,
     const double *__restrict__ cm, const int32_t *__restrict__ ring_pnum,
     const int32_t *__restrict__ ring_pden, const double2 *__restrict__ alm,
     double2 *__restrict__ F) {
-  const int m = blockIdx.x;
-  const int rp = blockIdx.y * blockDim.x + threadIdx.x;
-  const int rpc = rp < npairs ? rp : npairs - 1;
-  const double x = z[rpc];
-  double p0 = 0.0, p1;
-  int k;
-  legendre_seed(cm[m], sth[rpc], m, p1, k);
-
+  int m, rg;
+  if (!decode_m_run8(lmax, nrg, m, rg)) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int rp0 = (rg * (blockDim.x >> 6) + wave) * 64 * RPL + lane;
+  if (rp0 - lane >= npairs) return;  // wave-uniform; the kernel has no barriers
+  synth_state<RPL, NORM> s;
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) {
+    const int rp = min(rp0 + 64 * j, npairs - 1);
+    s.x[j] = z[rp];
+    s.p1[j] = 0.0;
+    legendre_seed_low(cm[m], sth[rp], m, s.p0[j], s.k[j]);
+    if (NORM) s.p0[j] = -s.p0[j];  // the first row's (gam = 0 / (1, -1)) yields the seed
+    s.acc[0][j] = s.acc[1][j] = double2{0.0, 0.0};
+  }
   const int64_t base = hp_index(lmax, m, m);
-  const double2 *__restrict__ a = alm + base;  // a[l - m]
-  const double2 *__restrict__ co = ab + base;  // co[l - m]
-  double er = 0.0, ei = 0.0, orr = 0.0, oi = 0.0;
-
-  int l = m;
-  // phase 1: some lane of the wave is still below the representable range
-  for (;;) {
-    if (l > m) {
-      const double2 c = co[l - m];
-      const double pn = c.x * (x * p1 - c.y * p0);
-      p0 = p1;
-      p1 = pn;
-    }
-    if (k < 0 && fabs(p1) > 0x1p300) { p1 *= 0x1p-600; p0 *= 0x1p-600; ++k; }
-    const double ve = (k == 0) ? p1 : 0.0;
-    double vo = 0.0;
-    if (l + 1 <= lmax) {
-      const double2 c = co[l + 1 - m];
-      const double pn = c.x * (x * p1 - c.y * p0);
-      p0 = p1;
-      p1 = pn;
-      if (k < 0 && fabs(p1) > 0x1p300) { p1 *= 0x1p-600; p0 *= 0x1p-600; ++k; }
-      vo = (k == 0) ? p1 : 0.0;
-    }
-    if (wave_any(k == 0)) {
-      const double2 ae = a[l - m];
-      er = fma(ve, ae.x, er);
-      ei = fma(ve, ae.y, ei);
-      if (l + 1 <= lmax) {
-        const double2 ao = a[l + 1 - m];
-        orr = fma(vo, ao.x, orr);
-        oi = fma(vo, ao.y, oi);
+  const double2 *__restrict__ a = alm + base;
+  const double *__restrict__ c = tab + (NORM ? 1 : 2) * base;
+  const int nl = lmax + 1 - m;
+  bool scaled = true;  // wave-uniform: some value of the wave may still be scaled
+  int i = 0;
+  for (; i + kRows <= nl; i += kRows) {
+    double2 cv[kRows], av[kRows];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) cv[q] = row_coef<NORM>(c, i + q);
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) av[q] = a[i + q];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) s.step(q & 1, cv[q], av[q]);
+    if (scaled && (i & kRows)) {
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < RPL; ++j) {
+        rescale_low(s.p0[j], s.p1[j], s.k[j]);
+        any |= s.k[j] < 0;
       }
+      scaled = wave_any(any);
     }
-    l += 2;
-    if (l > lmax || !wave_any(k < 0)) break;
   }
-  // phase 2: every lane in range, (l - m) even at the top of the loop
-  for (; l + 1 <= lmax; l += 2) {
-    const double2 c0 = co[l - m], c1 = co[l + 1 - m];
-    const double2 ae = a[l - m], ao = a[l + 1 - m];
-    double pn = c0.x * (x * p1 - c0.y * p0);
-    p0 = p1;
-    p1 = pn;
-    er = fma(p1, ae.x, er);
-    ei = fma(p1, ae.y, ei);
-    pn = c1.x * (x * p1 - c1.y * p0);
-    p0 = p1;
-    p1 = pn;
-    orr = fma(p1, ao.x, orr);
-    oi = fma(p1, ao.y, oi);
+  {  // the last rows (the turns leave i even), loaded together
+    double2 cv[kRows - 1], av[kRows - 1];
+#pragma unroll
+    for (int q = 0; q < kRows - 1; ++q) {
+      const int r = min(i + q, nl - 1);
+      cv[q] = row_coef<NORM>(c, r);
+      av[q] = a[r];
+    }
+#pragma unroll
+    for (int q = 0; q < kRows - 1; ++q)
+      if (i + q < nl) s.step(q & 1, cv[q], av[q]);
   }
-  if (l <= lmax) {
-    const double2 c0 = co[l - m];
-    const double2 ae = a[l - m];
-    const double pn = c0.x * (x * p1 - c0.y * p0);
-    p1 = pn;
-    er = fma(p1, ae.x, er);
-    ei = fma(p1, ae.y, ei);
-  }
-  if (m == 0) { ei = 0.0; oi = 0.0; }  // Im a_l0 is ignored (real map)
-  if (rp >= npairs) return;
-  // ring phase e^{i m phi0}, phi0 = 2 pi pnum / pden (the same on the south mirror)
-  const int pnum = ring_pnum[rp], pden = ring_pden[rp];
-  double ps = 0.0, pc = 1.0;
-  if (pnum) sincospi(2.0 * double((int64_t(m) * pnum) % pden) / double(pden), &ps, &pc);
+
   const int64_t stride = lmax + 1;
-  const double nr = er + orr, ni = ei + oi, sr = er - orr, si = ei - oi;
-  F[int64_t(rp) * stride + m] = double2{nr * pc - ni * ps, nr * ps + ni * pc};
-  if (rp < npairs - 1)
-    F[int64_t(nrings - 1 - rp) * stride + m] = double2{sr * pc - si * ps, sr * ps + si * pc};
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) {
+    const int rp = rp0 + 64 * j;
+    if (rp >= npairs) continue;
+    double2 e = s.acc[0][j], o = s.acc[1][j];
+    if (m == 0) e.y = o.y = 0.0;  // Im a_l0 is ignored (real map)
+    // ring phase e^{i m phi0}, phi0 = 2 pi pnum / pden (the same on the south mirror)
+    const int pnum = ring_pnum[rp], pden = ring_pden[rp];
+    double ps = 0.0, pc = 1.0;
+    if (pnum) sincospi(2.0 * double((int64_t(m) * pnum) % pden) / double(pden), &ps, &pc);
+    const double nr = e.x + o.x, ni = e.y + o.y, sr = e.x - o.x, si = e.y - o.y;
+    F[int64_t(rp) * stride + m] = double2{nr * pc - ni * ps, nr * ps + ni * pc};
+    if (rp < npairs - 1)
+      F[int64_t(nrings - 1 - rp) * stride + m] = double2{sr * pc - si * ps, sr * ps + si * pc};
+  }
+}
+
+__global__ __launch_bounds__(256) void scale_alm_kernel(int64_t n, const double2 *__restrict__ alm,
+                                                        const double *__restrict__ csc,
+                                                        double2 *__restrict__ out) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) out[i] = double2{alm[i].x * csc[i], alm[i].y * csc[i]};
+}
+
+template <int RPL, bool NORM>
+int launch(const ga_plan *p, const double *alm, double *F, hipStream_t stream) {
+  const int nw = std::min(4, (p->npairs + 64 * RPL - 1) / (64 * RPL));
+  const int nrg = (p->npairs + 64 * RPL * nw - 1) / (64 * RPL * nw);
+  hipLaunchKernelGGL((legendre_synth_f64_kernel<RPL, NORM>), dim3(m_run8_blocks(p->lmax, nrg)),
+                     dim3(64 * nw), 0, stream, p->lmax, p->npairs, p->nrings, nrg, p->d_z, p->d_sth,
+                     NORM ? p->d_gam : reinterpret_cast<const double *>(p->d_aab), p->d_cm,
+                     p->d_ring_pnum, p->d_ring_pden, reinterpret_cast<const double2 *>(alm),
+                     reinterpret_cast<double2 *>(F));
+  GA_LAUNCH_CHECK();
+  return GA_OK;
 }
 
 }  // namespace
 
-int launch_legendre_synth_f64(const ga_plan *p, const double *alm, double *F,
-                              hipStream_t stream) {
-  dim3 grid(unsigned(p->lmax + 1), unsigned((p->npairs + 255) / 256));
-  hipLaunchKernelGGL(legendre_synth_f64_kernel, grid, dim3(256), 0, stream, p->lmax, p->npairs,
-                     p->nrings, p->d_z, p->d_sth, p->d_ab, p->d_cm, p->d_ring_pnum,
-                     p->d_ring_pden, reinterpret_cast<const double2 *>(alm),
-                     reinterpret_cast<double2 *>(F));
+int launch_legendre_synth_f64(const ga_plan *p, const double *alm, double *F, double *scratch,
+                              size_t scratch_doubles, hipStream_t stream) {
+  // The normalised form saves an operation in five and, with two pairs per
+  // lane, half the scalar loads, but costs the launch of the scaling pass and
+  // the wait between the two, and half the waves.  Measured (whole alm2map):
+  // nside 256, lmax 512 (4104 waves of one pair per lane): plain 53.6 us,
+  // normalised 76; nside 512, lmax 1023 (16384 waves): 222 and 209 us; nside
+  // 1024, lmax 2048: 1232 and 1003 us.
+  const int64_t waves = int64_t(p->lmax + 1) * ((p->npairs + 63) / 64);
+  if (waves < kManyWaves || scratch_doubles < size_t(2 * p->nalm))
+    return launch<1, false>(p, alm, F, stream);
+  hipLaunchKernelGGL(scale_alm_kernel, dim3(unsigned((p->nalm + 255) / 256)), dim3(256), 0, stream,
+                     p->nalm, reinterpret_cast<const double2 *>(alm), p->d_csc,
+                     reinterpret_cast<double2 *>(scratch));
   GA_LAUNCH_CHECK();
-  return GA_OK;
+  return launch<2, true>(p, scratch, F, stream);
 }
 
 }  // namespace ga

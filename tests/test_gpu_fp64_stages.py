@@ -57,3 +57,18 @@ def test_analysis_edges(nside, lmax, niter):
     ref = O.map2alm(f, lmax, niter=niter, nthreads=8)
     got = hp.map2alm(f, lmax=lmax, iter=niter)
     assert np.max(np.abs(got - ref)) / np.sqrt(np.mean(np.abs(ref) ** 2)) < bound(lmax)
+
+
+# the plain form (few waves), the normalised one with two ring pairs per lane
+# (at least 16384 waves: nside 512, lmax 1030 and nside 520, lmax 1023 with a
+# part-filled last wave), and no room in the map for the scaled alm (lmax 600
+# at nside 40)
+@pytest.mark.parametrize("nside,lmax", [(1, 0), (1, 6), (2, 7), (33, 8), (64, 15), (65, 16),
+                                        (40, 600), (512, 1030), (520, 1023)])
+def test_synthesis_edges(nside, lmax):
+    print(f"synthesis nside={nside} lmax={lmax}", flush=True)
+    rng = np.random.default_rng(3 * nside + lmax)
+    alm = rand_alm(lmax, rng)
+    ref = O.alm2map(alm, nside, nthreads=8)
+    got = hp.alm2map(alm, nside)
+    assert np.max(np.abs(got - ref)) / np.sqrt(np.mean(ref**2)) < bound(lmax)
