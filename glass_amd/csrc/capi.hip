@@ -9,19 +9,18 @@
 namespace ga {
 namespace {
 
-template <typename T>
-__global__ void residual_kernel(int64_t n, const T *__restrict__ a, T *__restrict__ b) {
+__global__ void residual_kernel(int64_t n, const float *__restrict__ a, float *__restrict__ b) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) b[i] = a[i] - b[i];
 }
 
 // dst = src * w * c per pixel (dst may be src): the per-pixel quadrature
 // weights of a weighted analysis, c undoing the analysis's uniform 4 pi / npix
-template <typename T>
-__global__ void weight_pixels_kernel(int64_t n, int64_t npix, const T *__restrict__ src,
-                                     const double *__restrict__ w, double c, T *dst) {
+// (FP32; the FP64 ring stage weights the pixels in its load)
+__global__ void weight_pixels_kernel(int64_t n, int64_t npix, const float *__restrict__ src,
+                                     const double *__restrict__ w, double c, float *dst) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = T(double(src[i]) * (w[i % npix] * c));
+  if (i < n) dst[i] = float(double(src[i]) * (w[i % npix] * c));
 }
 
 // same size as ga_workspace_size: fp32 ring buffers hold whole groups of
@@ -74,7 +73,7 @@ extern "C" int ga_alm2map_f64(const ga_plan *p, const double *alm, double *map, 
   int rc = launch_legendre_synth_f64(p, alm, F, apart ? map : nullptr,
                                      apart ? size_t(p->npix) : 0, s);
   if (rc) return rc;
-  return launch_ring_synth_f64(p, 1, 1, F, map, nullptr, s);
+  return launch_ring_synth_f64(p, 1, F, map, nullptr, s);
 }
 
 extern "C" int ga_alm2map_batch_f32(const ga_plan *p, int32_t S, const float *alm, float *maps,
@@ -243,7 +242,9 @@ static int map2alm_impl(const ga_plan *p, int S, const T *map, T *alm, int niter
         rc = launch_legendre_synth_f64(p, (const double *)alm, (double *)F, (double *)map_tmp,
                                        size_t(p->npix), s);
         if (rc) return rc;
-        rc = launch_ring_synth_f64(p, 1, 1, (const double *)F, (double *)map_tmp, nullptr, s);
+        rc = launch_ring_synth_f64(p, 1, (const double *)F, (double *)map_tmp,
+                                   (const double *)map, s);
+        subtract = false;
       } else {
         rc = launch_legendre_synth_batch(p, S, (const float *)alm, ws, s);
         if (rc) return rc;
@@ -258,21 +259,21 @@ static int map2alm_impl(const ga_plan *p, int S, const T *map, T *alm, int niter
         }
       }
       if (rc) return rc;
-      if (subtract) {
-        hipLaunchKernelGGL(residual_kernel<T>, dim3(unsigned((npx + 255) / 256)), dim3(256), 0,
-                           s, npx, map, map_tmp);
+      if (subtract) {  // FP32 only
+        hipLaunchKernelGGL(residual_kernel, dim3(unsigned((npx + 255) / 256)), dim3(256), 0,
+                           s, npx, (const float *)map, (float *)map_tmp);
         GA_LAUNCH_CHECK();
       }
       src = map_tmp;
     }
-    if (pixw) {
-      hipLaunchKernelGGL(weight_pixels_kernel<T>, dim3(unsigned((npx + 255) / 256)), dim3(256), 0,
-                         s, npx, int64_t(p->npix), src, pixw, wc, map_tmp);
+    if (pixw && sizeof(T) == 4) {
+      hipLaunchKernelGGL(weight_pixels_kernel, dim3(unsigned((npx + 255) / 256)), dim3(256), 0, s,
+                         npx, int64_t(p->npix), (const float *)src, pixw, wc, (float *)map_tmp);
       GA_LAUNCH_CHECK();
       src = map_tmp;
     }
     if (sizeof(T) == 8) {
-      rc = launch_ring_anal_f64(p, S, (const double *)src, (double *)F, s);
+      rc = launch_ring_anal_f64(p, (const double *)src, pixw, wc, (double *)F, s);
       if (rc) return rc;
       rc = launch_legendre_anal_f64(p, (const double *)F, (double *)alm, (double *)partial, it > 0,
                                     s);
@@ -330,7 +331,7 @@ extern "C" int ga_alm2map_spin_f64(const ga_plan *p, int32_t spin, const double 
   hipStream_t s = (hipStream_t)stream;
   int rc = launch_spin_synth_f64(p, spin, E, B, (double *)ws, s);
   if (rc) return rc;
-  return launch_ring_synth_f64(p, 2, 2, (const double *)ws, maps, nullptr, s);
+  return launch_ring_synth_f64(p, 2, (const double *)ws, maps, nullptr, s);
 }
 
 extern "C" int ga_alm2map_spin_batch_f32(const ga_plan *p, int32_t spin, int32_t S,

@@ -63,13 +63,16 @@ int launch_legendre_contract_grouped(int ngroup, const ga_plan *const *plans, co
 // the shells in groups of G: offset ((ring ngrp + s/G)(lmax+1) + m) G + s%G
 // (G = S is the plain [ring][m][S] layout; the MFMA stages write
 // G = ring_group(S)).
-int launch_ring_synth_f64(const ga_plan *p, int S, int G, const double *F, double *maps,
-                          const ga_epilogue *epi, hipStream_t s);
+// FP64: S = 1 or 2 maps, F [ring][m][S]; with ref, maps = ref - synthesis
+int launch_ring_synth_f64(const ga_plan *p, int S, const double *F, double *maps,
+                          const double *ref, hipStream_t s);
 int launch_ring_synth_f32(const ga_plan *p, int S, int G, const float *F, float *maps,
                           const ga_epilogue *epi, hipStream_t s);
 
 // Ring stage of analysis: maps [S][npix] -> F [ring][m][S] (weighted, phase removed)
-int launch_ring_anal_f64(const ga_plan *p, int S, const double *maps, double *F, hipStream_t s);
+// (FP64: one map; with pixw, pixel p is first multiplied by pixw[p] wc)
+int launch_ring_anal_f64(const ga_plan *p, const double *maps, const double *pixw, double wc,
+                         double *F, hipStream_t s);
 int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, float *F, hipStream_t s);
 // out = ref - FP32 ring synthesis of F (fused-pass forms only; GA_ERR_UNSUPPORTED
 // with nothing launched otherwise)

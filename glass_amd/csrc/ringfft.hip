@@ -1,4 +1,4 @@
-// Per-ring Fourier stage of the HEALPix transforms (FP32 and FP64).
+// Per-ring Fourier stage of the HEALPix transforms (FP32).
 //
 // Every HEALPix ring holds n = 4 r pixels (r = i on polar ring i, r = nside on
 // the equatorial belt).  A workgroup handles one ring and a PAIR of maps: the
@@ -29,46 +29,11 @@
 #include "common.h"
 #include "device.h"
 #include "kernels.h"
+#include "ringfft.h"
 
 namespace ga {
 
 namespace {
-
-template <typename T>
-struct tab_t;
-template <>
-struct tab_t<float> {
-  using type = float2;
-};
-template <>
-struct tab_t<double> {
-  using type = double2;
-};
-
-template <typename T>
-__device__ __forceinline__ cplx<T> ld(const typename tab_t<T>::type *p, int64_t i) {
-  auto v = p[i];
-  return {v.x, v.y};
-}
-
-__device__ __forceinline__ int ilog2(int x) { return 31 - __clz(x); }
-
-// LDS work arrays insert one pad element after every 32 (8-byte complex floats
-// span all 64 banks every 32 elements), which removes the bank conflicts of
-// the short-span butterflies and of the bit-reversed scatter.
-__device__ __forceinline__ int pad(int i) { return i + (i >> 5); }
-__host__ __device__ inline int padded_len(int n) { return n + (n >> 5) + 1; }
-
-__device__ __forceinline__ cplx<float> expi_q(int64_t q, int64_t d, float) {
-  float s, c;
-  sincospif(2.0f * float(q) / float(d), &s, &c);
-  return {c, s};
-}
-__device__ __forceinline__ cplx<double> expi_q(int64_t q, int64_t d, double) {
-  double s, c;
-  sincospi(2.0 * double(q) / double(d), &s, &c);
-  return {c, s};
-}
 
 // In-place forward FFT (e^{-2 pi i}), natural order in, bit-reversed out, on P
 // arrays X + p ldx at once (one barrier per stage for all of them).
@@ -158,12 +123,6 @@ __device__ void fft_dit(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
     }
     __syncthreads();
   }
-}
-
-__device__ __forceinline__ int blu_len(int r) {
-  int L = 1;
-  while (L < 2 * r - 1) L <<= 1;
-  return L;
 }
 
 // Inverse length-r DFT of the values H[i][slot][p] (owned j1 = t + i NT) for
@@ -280,7 +239,6 @@ __device__ __forceinline__ float expm1_map(float x) {
   return r;
 }
 __device__ __forceinline__ float expm1_t(float x) { return expm1_map(x); }
-__device__ __forceinline__ double expm1_t(double x) { return expm1(x); }
 
 template <typename T>
 __device__ __forceinline__ T apply_epi(T x, int kind, T lam, T par) {
@@ -645,203 +603,6 @@ __global__ __launch_bounds__(NT) void ring_anal_kernel(
 // bit-reversed chirp spectrum, inverse decimation in time.  The two ring
 // classes are launched separately (ring lists), each with LDS for its own
 // transform length.
-
-// e^{2 pi i k / 16} for k = 0..15: cos and sin
-__device__ __forceinline__ float c16(int k) {
-  switch (k & 15) {
-    case 0: return 1.0f;
-    case 1: case 15: return 0.92387953251128674f;
-    case 2: case 14: return 0.70710678118654752f;
-    case 3: case 13: return 0.38268343236508977f;
-    case 4: case 12: return 0.0f;
-    case 5: case 11: return -0.38268343236508977f;
-    case 6: case 10: return -0.70710678118654752f;
-    case 7: case 9: return -0.92387953251128674f;
-    default: return -1.0f;
-  }
-}
-__device__ __forceinline__ float s16(int k) { return c16(k - 4); }
-
-// v e^{SIGN 2 pi i k / 16} (k a compile-time constant after unrolling)
-template <int SIGN>
-__device__ __forceinline__ cplx<float> rot16(cplx<float> v, int k) {
-  k &= 15;
-  if (k == 0) return v;
-  if (k == 4) return SIGN > 0 ? cplx<float>{-v.im, v.re} : cplx<float>{v.im, -v.re};
-  if (k == 8) return cplx<float>{-v.re, -v.im};
-  if (k == 12) return SIGN > 0 ? cplx<float>{v.im, -v.re} : cplx<float>{-v.im, v.re};
-  const float c = c16(k), sn = SIGN * s16(k);
-  return cplx<float>{v.re * c - v.im * sn, v.re * sn + v.im * c};
-}
-
-__device__ __forceinline__ cplx<float> twid(const float2 *__restrict__ tw, int idx, int sign) {
-  const float2 w = tw[idx];
-  return cplx<float>{w.x, sign * w.y};
-}
-
-// One pass fusing K radix-2 stages with half-spans h0, 2 h0, .., 2^(K-1) h0
-// (DIT: stages in increasing span; DIF: decreasing) on A arrays of length N.
-// Group = elements base + q h0 (q < 2^K), base = blk 2^K h0 + b, b < h0.
-// A group either lies inside one 32-element block or starts on a multiple of
-// 32 with h0 dividing 32 or a multiple of it, so its padded slots are
-//   pad(base + q h0) = pad(base) + q h0 + (q h0 >> 5),
-// offsets that are the same for every thread of the pass.  tw holds
-// e^{2 pi i j / 2^ltw}.
-template <int K, int NT, bool DIT, int SIGN>
-__device__ __forceinline__ void fused_pass(cplx<float> *X, int ldx, int A, int N, int h0,
-                                           const float2 *__restrict__ tw, int ltw) {
-  constexpr int R = 1 << K;
-  const int lh0 = ilog2(h0);
-  const int lg = ilog2(N) - K;  // groups per array = N / R
-  const int total = A << lg;
-  int off[R];
-#pragma unroll
-  for (int q = 0; q < R; ++q) off[q] = (q << lh0) + ((q << lh0) >> 5);
-  for (int gg = threadIdx.x; gg < total; gg += NT) {
-    const int a = gg >> lg, g = gg & ((1 << lg) - 1);
-    const int b = g & (h0 - 1), blk = g >> lh0;
-    const int base = (blk << (K + lh0)) + b;
-    cplx<float> *Y = X + a * ldx + pad(base);
-    cplx<float> v[R];
-#pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = Y[off[q]];
-    // ws[s] = e^{SIGN 2 pi i b / (2^(s+1) h0)}: one table value per stage
-    cplx<float> ws[K];
-#pragma unroll
-    for (int s = 0; s < K; ++s) ws[s] = twid(tw, b << (ltw - s - 1 - lh0), SIGN);
-#pragma unroll
-    for (int ss = 0; ss < K; ++ss) {
-      const int s = DIT ? ss : K - 1 - ss;
-      const int d = 1 << s;
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        if (q & d) continue;
-        // twiddle of this pair: ws[s] e^{SIGN 2 pi i (q mod d) / (2 d)}
-        const cplx<float> t = rot16<SIGN>(ws[s], (q & (d - 1)) * (16 >> (s + 1)));
-        if (DIT) {
-          const cplx<float> y = cmul(v[q + d], t);
-          const cplx<float> x = v[q];
-          v[q] = cadd(x, y);
-          v[q + d] = csub(x, y);
-        } else {
-          const cplx<float> x = v[q], y = v[q + d];
-          v[q] = cadd(x, y);
-          v[q + d] = cmul(csub(x, y), t);
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) Y[off[q]] = v[q];
-  }
-  __syncthreads();
-}
-
-// full power-of-two transform of A arrays: DIT (bit-reversed in, natural out)
-// or DIF (natural in, bit-reversed out)
-template <int NT, bool DIT, int SIGN>
-__device__ __forceinline__ void fused_fft(cplx<float> *X, int ldx, int A, int N,
-                                          const float2 *__restrict__ tw, int twlen) {
-  const int lN = ilog2(N), ltw = ilog2(twlen);
-  if (DIT) {
-    for (int l = 0; l < lN;) {
-      const int K = lN - l >= 4 ? 4 : lN - l;
-      switch (K) {
-        case 4: fused_pass<4, NT, true, SIGN>(X, ldx, A, N, 1 << l, tw, ltw); break;
-        case 3: fused_pass<3, NT, true, SIGN>(X, ldx, A, N, 1 << l, tw, ltw); break;
-        case 2: fused_pass<2, NT, true, SIGN>(X, ldx, A, N, 1 << l, tw, ltw); break;
-        default: fused_pass<1, NT, true, SIGN>(X, ldx, A, N, 1 << l, tw, ltw); break;
-      }
-      l += K;
-    }
-  } else {
-    for (int l = lN; l > 0;) {  // stages with half-spans 2^(l-1) down to 1
-      const int K = l >= 4 ? 4 : l;
-      const int h0 = 1 << (l - K);
-      switch (K) {
-        case 4: fused_pass<4, NT, false, SIGN>(X, ldx, A, N, h0, tw, ltw); break;
-        case 3: fused_pass<3, NT, false, SIGN>(X, ldx, A, N, h0, tw, ltw); break;
-        case 2: fused_pass<2, NT, false, SIGN>(X, ldx, A, N, h0, tw, ltw); break;
-        default: fused_pass<1, NT, false, SIGN>(X, ldx, A, N, h0, tw, ltw); break;
-      }
-      l -= K;
-    }
-  }
-}
-
-// The middle of a Bluestein convolution as one pass: the last forward DIF
-// pass (K stages, half-spans 2^(K-1) .. 1), the product with the chirp
-// spectrum (stored bit-reversed, i.e. in the order the DIF leaves the
-// values) and the first inverse DIT pass (half-spans 1 .. 2^(K-1)) act on the
-// same groups of 2^K consecutive elements, whose twiddles are the constant
-// rotations alone; one LDS round trip instead of three.
-template <int K, int NT>
-__device__ __forceinline__ void mid_pass(cplx<float> *X, int ldx, int A, int L,
-                                         const float2 *__restrict__ bspec) {
-  constexpr int R = 1 << K;
-  const int lg = ilog2(L) - K;
-  const int total = A << lg;
-  for (int gg = threadIdx.x; gg < total; gg += NT) {
-    const int a = gg >> lg, g = gg & ((1 << lg) - 1);
-    const int base = g << K;
-    cplx<float> *Y = X + a * ldx + pad(base);  // a group never straddles a pad
-    cplx<float> v[R];
-#pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = Y[q];
-#pragma unroll
-    for (int s = K - 1; s >= 0; --s) {
-      const int d = 1 << s;
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        if (q & d) continue;
-        const cplx<float> tq = rot16<-1>(cplx<float>{1.0f, 0.0f}, (q & (d - 1)) * (16 >> (s + 1)));
-        const cplx<float> x = v[q], y = v[q + d];
-        v[q] = cadd(x, y);
-        v[q + d] = cmul(csub(x, y), tq);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const float2 b = bspec[base + q];
-      v[q] = cmul(v[q], cplx<float>{b.x, b.y});
-    }
-#pragma unroll
-    for (int s = 0; s < K; ++s) {
-      const int d = 1 << s;
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        if (q & d) continue;
-        const cplx<float> tq = rot16<1>(cplx<float>{1.0f, 0.0f}, (q & (d - 1)) * (16 >> (s + 1)));
-        const cplx<float> y = cmul(v[q + d], tq);
-        const cplx<float> x = v[q];
-        v[q] = cadd(x, y);
-        v[q + d] = csub(x, y);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) Y[q] = v[q];
-  }
-  __syncthreads();
-}
-
-// Bluestein convolution of A arrays of length L = 2^lN in place: forward DIF
-// passes (K = 4, half-spans down to 2^(l0)), the middle pass (K = l0 <= 4,
-// with the chirp spectrum), inverse DIT passes mirroring the forward ones;
-// natural order in and out.
-template <int NT>
-__device__ __forceinline__ void bluestein_conv(cplx<float> *X, int ldx, int A, int L,
-                                               const float2 *__restrict__ tw, int twlen,
-                                               const float2 *__restrict__ bspec) {
-  const int lN = ilog2(L), ltw = ilog2(twlen);
-  int l = lN;
-  for (; l > 4; l -= 4) fused_pass<4, NT, false, -1>(X, ldx, A, L, 1 << (l - 4), tw, ltw);
-  switch (l) {
-    case 4: mid_pass<4, NT>(X, ldx, A, L, bspec); break;
-    case 3: mid_pass<3, NT>(X, ldx, A, L, bspec); break;
-    case 2: mid_pass<2, NT>(X, ldx, A, L, bspec); break;
-    default: mid_pass<1, NT>(X, ldx, A, L, bspec); break;
-  }
-  for (int lo = l; lo < lN; lo += 4) fused_pass<4, NT, true, 1>(X, ldx, A, L, 1 << lo, tw, ltw);
-}
 
 // The aliasing fold of one ring's coefficients into its n = 4 r bins, for a
 // unit of two shells (h = G(s) + i G(s + 1)), written to the bin slots of X
@@ -1986,11 +1747,8 @@ int launch_ring_synth2_f32(const ga_plan *p, int S, int G, const float *F, float
 template <typename T>
 int launch_ring(const ga_plan *p, int S, int G, const void *in, void *out, const ga_epilogue *epi,
                 bool anal, hipStream_t stream) {
-  using tab = typename tab_t<T>::type;
-  const tab *blu = reinterpret_cast<const tab *>(sizeof(T) == 8 ? (const void *)p->d_blu64
-                                                               : (const void *)p->d_blu32);
-  const tab *tw = reinterpret_cast<const tab *>(sizeof(T) == 8 ? (const void *)p->d_tw64
-                                                              : (const void *)p->d_tw32);
+  static_assert(sizeof(T) == 4, "the FP64 ring stages are in ringfft64.hip");
+  const float2 *blu = p->d_blu32, *tw = p->d_tw32;
   const int max_r = p->max_r;
   if (anal) {
     const int npp = (S + 1) / 2;
@@ -2063,10 +1821,6 @@ int launch_ring(const ga_plan *p, int S, int G, const void *in, void *out, const
 
 }  // namespace
 
-int launch_ring_synth_f64(const ga_plan *p, int S, int G, const double *F, double *maps,
-                          const ga_epilogue *epi, hipStream_t s) {
-  return launch_ring<double>(p, S, G, F, maps, epi, false, s);
-}
 int launch_ring_synth_f32(const ga_plan *p, int S, int G, const float *F, float *maps,
                           const ga_epilogue *epi, hipStream_t s) {
   if (p->tune.ring_path != 1) {
@@ -2087,9 +1841,6 @@ int launch_ring_resid_f32(const ga_plan *p, int S, int G, const float *F, float 
   const int rc = launch_ring_synth2_f32(p, S, G, F, out, nullptr, p->tune.ring_path != 2, s, ref);
   if (rc == GA_ERR_UNSUPPORTED) clear_error();
   return rc;
-}
-int launch_ring_anal_f64(const ga_plan *p, int S, const double *maps, double *F, hipStream_t s) {
-  return launch_ring<double>(p, S, S, maps, F, nullptr, true, s);
 }
 int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, float *F, hipStream_t s) {
   if (p->tune.ring_path != 1) {

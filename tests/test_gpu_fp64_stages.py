@@ -72,3 +72,18 @@ def test_synthesis_edges(nside, lmax):
     ref = O.alm2map(alm, nside, nthreads=8)
     got = hp.alm2map(alm, nside)
     assert np.max(np.abs(got - ref)) / np.sqrt(np.mean(ref**2)) < bound(lmax)
+
+
+def test_synthesis_longest_rings():
+    """Rings of more than 4 * 2048 pixels (eight values of a thread), both for
+    a power of two and for Bluestein lengths above 4096."""
+    nside, lmax = 2100, 12
+    rng = np.random.default_rng(5)
+    alm = rand_alm(lmax, rng)
+    got = hp.alm2map(alm, nside)
+    first, step = 1, 419  # a sample of rings through the oracle
+    ref = O.alm2map_rings(alm, nside, first, step, nthreads=8)
+    sel = ref != 0
+    assert sel.sum() > nside
+    err = np.max(np.abs(got[sel] - ref[sel])) / np.sqrt(np.mean(ref[sel] ** 2))
+    assert err < bound(lmax)
