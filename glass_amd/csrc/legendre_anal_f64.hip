@@ -32,54 +32,7 @@ namespace {
 
 constexpr int kRows = 16;        // l rows per reduction
 constexpr int kSums = 2 * kRows;  // (re, im) of each
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v) {
-  const uint64_t u = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(u)), CTRL, 0xF, 0xF, false);
-  const uint32_t hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(u >> 32)), CTRL, 0xF, 0xF, false);
-  return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
-}
-// lanes with `bit` unset get a summed over the lane and its partner, the
-// others b; the partner (CTRL) has the other `bit`
-template <int CTRL>
-__device__ __forceinline__ double halve(double a, double b, bool bit) {
-  const double keep = bit ? b : a, send = bit ? a : b;
-  return keep + dpp_move<CTRL>(send);
-}
-template <bool ROWS16>
-__device__ __forceinline__ double halve_swap(double a, double b) {
-  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
-  // (X, Y) -> ([X_lo | Y_lo], [X_hi | Y_hi]) over halves of the wave, or over
-  // even and odd rows of 16 lanes
-  uint32_t l0, l1, h0, h1;
-  if (ROWS16) {
-    const auto l = __builtin_amdgcn_permlane16_swap(uint32_t(ua), uint32_t(ub), false, false);
-    const auto h = __builtin_amdgcn_permlane16_swap(uint32_t(ua >> 32), uint32_t(ub >> 32), false, false);
-    l0 = l[0]; l1 = l[1]; h0 = h[0]; h1 = h[1];
-  } else {
-    const auto l = __builtin_amdgcn_permlane32_swap(uint32_t(ua), uint32_t(ub), false, false);
-    const auto h = __builtin_amdgcn_permlane32_swap(uint32_t(ua >> 32), uint32_t(ub >> 32), false, false);
-    l0 = l[0]; l1 = l[1]; h0 = h[0]; h1 = h[1];
-  }
-  return __builtin_bit_cast(double, (uint64_t(h0) << 32) | l0) +
-         __builtin_bit_cast(double, (uint64_t(h1) << 32) | l1);
-}
-
-// the 32 sums v[0..31] over the 64 lanes: lane L returns sum L / 2
-__device__ __forceinline__ double wave_sums32(const double (&v)[kSums], int lane) {
-  double a[16], b[8], c[4], d[2];
-#pragma unroll
-  for (int q = 0; q < 16; ++q) a[q] = halve_swap<false>(v[q], v[q + 16]);
-#pragma unroll
-  for (int q = 0; q < 8; ++q) b[q] = halve_swap<true>(a[q], a[q + 8]);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) c[q] = halve<0x128>(b[q], b[q + 4], lane & 8);  // row_ror:8
-#pragma unroll
-  for (int q = 0; q < 2; ++q) d[q] = halve<0x141>(c[q], c[q + 2], lane & 4);  // row_half_mirror
-  const double e = halve<0x1B>(d[0], d[1], lane & 2);                          // quad_perm [3,2,1,0]
-  return e + dpp_move<0xB1>(e);                                                // quad_perm [1,0,3,2]
-}
+static_assert(kSums == 32, "wave_sums32");
 
 template <int RPL>
 __global__ __launch_bounds__(256, RPL == 8 ? 2 : 3) void legendre_anal_f64_kernel(

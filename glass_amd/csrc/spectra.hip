@@ -9,9 +9,9 @@
 // With n Gauss-Legendre nodes (x_k, w_k) and n coefficients l < n the pair is
 // exact (products P_l P_l' of degree < 2n - 1 are integrated exactly), so
 // corr2cl(cl2corr(cl)) = cl to rounding.  P_l by its three-term recurrence in
-// FP64, one thread per node; corr2cl reduces each l over the 64 nodes of a
-// wave (xor butterfly) and then over waves in a fixed order, so the result
-// does not depend on scheduling.  The nodes come from Newton's method on P_n
+// FP64, one lane per node; corr2cl reduces 32 l at a time over the 64 nodes of
+// a wave and then over waves in a fixed order, so the result does not depend
+// on scheduling.  The nodes come from Newton's method on P_n
 // from the asymptotic first guess cos(pi (i + 3/4) / (n + 1/2)), one thread
 // per node pair (x, -x).
 #include "common.h"
@@ -57,61 +57,122 @@ __global__ __launch_bounds__(256) void gl_nodes_kernel(int n, double *__restrict
   if ((n & 1) && i == n / 2) x[i] = 0.0;
 }
 
-__global__ __launch_bounds__(256) void cl2corr_kernel(int nl, const double *__restrict__ cl,
-                                                      int n, const double *__restrict__ x,
-                                                      double *__restrict__ corr) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const double xk = x[k];
-  double p0 = 1.0, p1 = xk;
-  double acc = cl[0] * (1.0 / (4.0 * M_PI));
-  if (nl > 1) acc += cl[1] * (3.0 / (4.0 * M_PI)) * xk;
-  for (int l = 2; l < nl; ++l) {
-    const double p2 = (double(2 * l - 1) * xk * p1 - double(l - 1) * p0) / double(l);
-    p0 = p1;
-    p1 = p2;
-    acc += cl[l] * (double(2 * l + 1) / (4.0 * M_PI)) * p2;
-  }
-  corr[k] = acc;
+// Rows of the recurrence P_l = (a_l x) P_{l-1} - b_l P_{l-2}, a_l = (2l-1)/l, b_l =
+// (l-1)/l, for kChunk values of l at a time: lane i works out row l0 + i (its
+// divisions would otherwise be done by every lane in every step) into LDS,
+// from where all lanes read it; the row of l = 0, (0, -1), yields P_0 = 1 from
+// (P_{-2}, P_{-1}) = (1, 0).
+__device__ __forceinline__ double2 legendre_row(int l) {
+  return l == 0 ? double2{0.0, -1.0} : double2{double(2 * l - 1) / l, double(l - 1) / l};
+}
+__device__ __forceinline__ double legendre_step(double2 ab, double x, double &p0, double &p1) {
+  const double p = fma(ab.x * x, p1, -(ab.y * p0));
+  p0 = p1;
+  p1 = p;
+  return p;
 }
 
-// part[wave][l]: 2 pi sum over the wave's nodes of w_k corr_k P_l(x_k)
-__global__ __launch_bounds__(256) void corr2cl_kernel(int n, const double *__restrict__ x,
-                                                      const double *__restrict__ w,
-                                                      const double *__restrict__ corr, int nl,
-                                                      int nwaves, double *__restrict__ part) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int wave = k >> 6, lane = k & 63;
-  if (wave >= nwaves) return;  // whole waves past the last row
+// One wave, 64 nodes.  Bound: the serial recurrence (one wave on each of n / 64
+// CUs, four FP64 operations a step): 123 us at nl = n = 6147, where the division in
+// every step and a load of cl_l waited for in it took 823 us.
+__global__ __launch_bounds__(64) void cl2corr_kernel(int nl, const double *__restrict__ cl, int n,
+                                                     const double *__restrict__ x,
+                                                     double *__restrict__ corr) {
+  __shared__ double2 ab[2][64];
+  __shared__ double c[2][64];
+  const int lane = threadIdx.x, k = blockIdx.x * 64 + lane;
+  const double xk = x[min(k, n - 1)];
+  auto fill = [&](int buf, int l0) {
+    const int l = l0 + lane;
+    ab[buf][lane] = legendre_row(l);
+    c[buf][lane] = l < nl ? cl[l] * (double(2 * l + 1) / (4.0 * M_PI)) : 0.0;
+  };
+  double p0 = 1.0, p1 = 0.0, acc = 0.0;
+  int buf = 0;
+  fill(0, 0);
+  __syncthreads();
+  for (int l0 = 0; l0 < nl; l0 += 64, buf ^= 1) {
+    if (l0 + 64 < nl) fill(buf ^ 1, l0 + 64);
+    // 16 rows to registers while the 16 before them are run: a wave that is
+    // alone on its CU hides no latency; rows past nl have c = 0
+    double2 r[4][16];
+    double cv[4][16];
+#pragma unroll
+    for (int q = 0; q <= 4; ++q) {
+      if (q < 4) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          r[q][j] = ab[buf][16 * q + j];
+          cv[q][j] = c[buf][16 * q + j];
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (q > 0) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          acc = fma(cv[q - 1][j], legendre_step(r[q - 1][j], xk, p0, p1), acc);
+      }
+    }
+    __syncthreads();
+  }
+  if (k < n) corr[k] = acc;
+}
+
+// part[wave][l]: 2 pi sum over the wave's nodes of w_k corr_k P_l(x_k), 32 rows
+// of l reduced over the wave at a time.  Bound as above, the reduction adding
+// half: 165 us at n = nl = 6147 (a shuffle butterfly for every l: 2076 us).
+__global__ __launch_bounds__(64) void corr2cl_kernel(int n, const double *__restrict__ x,
+                                                     const double *__restrict__ w,
+                                                     const double *__restrict__ corr, int nl,
+                                                     double *__restrict__ part) {
+  __shared__ double2 ab[2][32];
+  const int lane = threadIdx.x, k = blockIdx.x * 64 + lane;
   const bool ok = k < n;
   const double xk = ok ? x[k] : 0.0;
   const double a = ok ? 2.0 * M_PI * w[k] * corr[k] : 0.0;
-  double p0 = 1.0, p1 = xk;
-  double *__restrict__ out = part + int64_t(wave) * nl;
-  for (int l = 0; l < nl; ++l) {
-    double P;
-    if (l == 0) {
-      P = 1.0;
-    } else if (l == 1) {
-      P = xk;
-    } else {
-      P = (double(2 * l - 1) * xk * p1 - double(l - 1) * p0) / double(l);
-      p0 = p1;
-      p1 = P;
-    }
-    double v = a * P;
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    if (lane == 0) out[l] = v;
+  double *__restrict__ out = part + int64_t(blockIdx.x) * nl;
+  auto fill = [&](int buf, int l0) {
+    if (lane < 32) ab[buf][lane] = legendre_row(l0 + lane);
+  };
+  double p0 = 1.0, p1 = 0.0;
+  int buf = 0;
+  double2 r[32];  // rows 0..15 of a turn are loaded before the reduction of the last one
+  fill(0, 0);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; ++j) r[j] = ab[0][j];
+  for (int l0 = 0; l0 < nl; l0 += 32) {
+#pragma unroll
+    for (int j = 16; j < 32; ++j) r[j] = ab[buf][j];
+    buf ^= 1;
+    fill(buf, l0 + 32);
+    __builtin_amdgcn_sched_barrier(0);
+    double v[32];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) v[j] = a * legendre_step(r[j], xk, p0, p1);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) r[j] = ab[buf][j];
+    __builtin_amdgcn_sched_barrier(0);
+    const double s = wave_sums32(v, lane);
+    const int l = l0 + (lane >> 1);
+    if (!(lane & 1) && l < nl) out[l] = s;
   }
 }
 
-__global__ void corr2cl_sum_kernel(int nl, int nwaves, const double *__restrict__ part,
-                                   double *__restrict__ cl) {
-  const int l = blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= nl) return;
+// cl[l] = the waves' parts, four interleaved sums added in order
+__global__ __launch_bounds__(256) void corr2cl_sum_kernel(int nl, int nwaves,
+                                                          const double *__restrict__ part,
+                                                          double *__restrict__ cl) {
+  __shared__ double red[4][64];
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int l = blockIdx.x * 64 + lane;
   double acc = 0.0;
-  for (int wv = 0; wv < nwaves; ++wv) acc += part[int64_t(wv) * nl + l];
-  cl[l] = acc;
+  if (l < nl)
+    for (int wv = g; wv < nwaves; wv += 4) acc += part[int64_t(wv) * nl + l];
+  red[g][lane] = acc;
+  __syncthreads();
+  if (g == 0 && l < nl) cl[l] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
 }  // namespace
@@ -133,7 +194,7 @@ extern "C" int ga_cl2corr(int32_t nl, const double *cl, int32_t n, const double 
                           void *stream) {
   clear_error();
   GA_REQUIRE(nl >= 1 && n >= 1 && cl && x && corr, GA_ERR_INVALID, "invalid argument");
-  hipLaunchKernelGGL(cl2corr_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, nl,
+  hipLaunchKernelGGL(cl2corr_kernel, dim3((n + 63) / 64), dim3(64), 0, (hipStream_t)stream, nl,
                      cl, n, x, corr);
   GA_LAUNCH_CHECK();
   return GA_OK;
@@ -155,10 +216,9 @@ extern "C" int ga_corr2cl(int32_t n, const double *x, const double *w, const dou
   GA_REQUIRE(ws_bytes >= need, GA_ERR_WORKSPACE, "workspace %zu < %zu bytes", ws_bytes, need);
   hipStream_t s = (hipStream_t)stream;
   double *part = static_cast<double *>(ws);
-  hipLaunchKernelGGL(corr2cl_kernel, dim3((nwaves * 64 + 255) / 256), dim3(256), 0, s, n, x, w,
-                     corr, nl, nwaves, part);
+  hipLaunchKernelGGL(corr2cl_kernel, dim3(nwaves), dim3(64), 0, s, n, x, w, corr, nl, part);
   GA_LAUNCH_CHECK();
-  hipLaunchKernelGGL(corr2cl_sum_kernel, dim3((nl + 255) / 256), dim3(256), 0, s, nl, nwaves, part,
+  hipLaunchKernelGGL(corr2cl_sum_kernel, dim3((nl + 63) / 64), dim3(256), 0, s, nl, nwaves, part,
                      cl);
   GA_LAUNCH_CHECK();
   return GA_OK;

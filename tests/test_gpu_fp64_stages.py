@@ -8,13 +8,18 @@ perturbations of lmax steps add, so max |error| / RMS of the oracle's result
 stays below 64 (lmax + 1) 2^-52.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
+import torch
+from scipy.special import eval_legendre
 
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
+from glass_amd import _lib  # noqa: E402
 from glass_amd import healpix as hp  # noqa: E402
 
 
@@ -87,3 +92,30 @@ def test_synthesis_longest_rings():
     assert sel.sum() > nside
     err = np.max(np.abs(got[sel] - ref[sel])) / np.sqrt(np.mean(ref[sel] ** 2))
     assert err < bound(lmax)
+
+
+@pytest.mark.parametrize("nl,n", [(1, 64), (2, 3), (16, 65), (33, 63), (64, 64), (65, 130), (97, 40),
+                                  (200, 129)])
+def test_transforms_of_unequal_lengths(nl, n):
+    """nl coefficients on n nodes around whole batches of rows (16, 32, 64) and
+    whole waves of nodes, against direct sums over scipy's Legendre
+    polynomials; tolerance: nl steps of a few ulp, 16 nl 2^-52 of the sum of
+    absolute terms."""
+    rng = np.random.default_rng(nl * 1000 + n)
+    x = np.sort(rng.uniform(-1, 1, n))
+    w, cl, corr = rng.uniform(0, 1, n), rng.standard_normal(nl), rng.standard_normal(n)
+    P = np.array([eval_legendre(l, x) for l in range(nl)])
+    dev = [torch.as_tensor(v).cuda() for v in (x, w, cl, corr)]
+    out_c = torch.empty(n, dtype=torch.float64, device="cuda")
+    out_l = torch.empty(nl, dtype=torch.float64, device="cuda")
+    _lib.call("ga_cl2corr", nl, _lib.ptr(dev[2]), n, _lib.ptr(dev[0]), _lib.ptr(out_c),
+              _lib.stream_ptr())
+    nb = ctypes.c_size_t()
+    _lib.call("ga_corr2cl_workspace_size", n, nl, ctypes.byref(nb))
+    ws = _lib.workspace(nb.value)
+    _lib.call("ga_corr2cl", n, _lib.ptr(dev[0]), _lib.ptr(dev[1]), _lib.ptr(dev[3]), nl,
+              _lib.ptr(out_l), _lib.ptr(ws), ws.numel(), _lib.stream_ptr())
+    f = (2 * np.arange(nl) + 1) / (4 * np.pi) * cl
+    assert np.all(np.abs(out_c.cpu().numpy() - f @ P) <= 16 * nl * 2.0**-52 * np.sum(np.abs(f)))
+    g = 2 * np.pi * w * corr
+    assert np.all(np.abs(out_l.cpu().numpy() - P @ g) <= 16 * nl * 2.0**-52 * np.sum(np.abs(g)))
