@@ -12,9 +12,13 @@ namespace ga {
 
 namespace {
 
-// healpy index i -> (l, m) for mmax = lmax = L:  i = m (2L + 1 - m) / 2 + l
+// healpy index i -> (l, m) for mmax = lmax = L:  i = m (2L + 1 - m) / 2 + l.  m is
+// the largest with hp_index(m, m) = m (2L + 3 - m) / 2 <= i; the loops only mend the
+// rounding of the root (one step at most; solving with 2L + 1 instead, the row
+// before its diagonal, overshoots by up to sqrt(2L) near m = L, and the loop back
+// made almxfl of 132k coefficients take 47 us instead of 4).
 __device__ __forceinline__ void hp_decode(int64_t i, int L, int &l, int &m) {
-  const double b = 2.0 * L + 1.0;
+  const double b = 2.0 * L + 3.0;
   int mm = int((b - sqrt(b * b - 8.0 * double(i))) * 0.5);
   if (mm < 0) mm = 0;
   while (mm > 0 && hp_index(L, mm, mm) > i) --mm;

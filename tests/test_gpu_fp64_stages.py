@@ -119,3 +119,14 @@ def test_transforms_of_unequal_lengths(nl, n):
     assert np.all(np.abs(out_c.cpu().numpy() - f @ P) <= 16 * nl * 2.0**-52 * np.sum(np.abs(f)))
     g = 2 * np.pi * w * corr
     assert np.all(np.abs(out_l.cpu().numpy() - P @ g) <= 16 * nl * 2.0**-52 * np.sum(np.abs(g)))
+
+
+@pytest.mark.parametrize("nl", [1, 2, 3, 64, 257, 1500])
+def test_alm_order(nl):
+    """(l, m) of every healpy index: the reordered index itself comes back."""
+    g = np.arange(nl * (nl + 1) // 2)
+    a = torch.as_tensor(g.astype(np.complex128)).cuda()
+    out = torch.empty_like(a)
+    _lib.call("ga_glass_to_healpix_alm_f64", nl, _lib.ptr(a), _lib.ptr(out), _lib.stream_ptr())
+    ref = np.concatenate([np.arange(m, nl) * (np.arange(m, nl) + 1) // 2 + m for m in range(nl)])
+    np.testing.assert_array_equal(out.cpu().numpy().real, ref)
