@@ -121,6 +121,33 @@ def test_transforms_of_unequal_lengths(nl, n):
     assert np.all(np.abs(out_l.cpu().numpy() - P @ g) <= 16 * nl * 2.0**-52 * np.sum(np.abs(g)))
 
 
+@pytest.mark.parametrize("k", range(9))
+def test_iternorm_row_lengths(k):
+    """Every row length of the register form (k <= 7) and the first of the
+    general one, in two calls that hand the state over, for 1 and 70 modes."""
+    rng = np.random.default_rng(k)
+    n = 2 * k + 5
+    for nl in (1, 70):
+        a = rng.standard_normal((nl, n, n + 3))
+        full = a @ a.transpose(0, 2, 1) / (n + 3) + np.eye(n)
+        rows = np.zeros((n, nl, k + 1))
+        for t in range(n):
+            for d in range(min(k, t) + 1):
+                rows[t, :, d] = full[:, t, t - d] * (1.0 if d == 0 else 0.5**d)
+        ref = list(O.iternorm(list(rows)))
+        m = ctypes.c_int32()
+        _lib.call("ga_iternorm_state_doubles", k, ctypes.byref(m))
+        state = torch.empty(nl * m.value, dtype=torch.float64, device="cuda")
+        flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+        cov = torch.as_tensor(rows).cuda()
+        w = torch.empty_like(cov)
+        for lo, hi in ((0, k + 2), (k + 2, n)):
+            _lib.call("ga_iternorm_batch", nl, k, k, k, hi - lo, int(lo == 0), _lib.ptr(cov[lo]),
+                      _lib.ptr(state), _lib.ptr(w[lo]), _lib.ptr(flag), _lib.stream_ptr())
+        assert not int(flag.item())
+        np.testing.assert_allclose(w.cpu().numpy(), np.array(ref), rtol=1e-12, atol=1e-12)
+
+
 @pytest.mark.parametrize("nl", [1, 2, 3, 64, 257, 1500])
 def test_alm_order(nl):
     """(l, m) of every healpy index: the reordered index itself comes back."""
