@@ -266,19 +266,21 @@ static int map2alm_impl(const ga_plan *p, int S, const T *map, T *alm, int niter
       }
       src = map_tmp;
     }
-    if (pixw && sizeof(T) == 4) {
-      hipLaunchKernelGGL(weight_pixels_kernel, dim3(unsigned((npx + 255) / 256)), dim3(256), 0, s,
-                         npx, int64_t(p->npix), (const float *)src, pixw, wc, (float *)map_tmp);
-      GA_LAUNCH_CHECK();
-      src = map_tmp;
-    }
     if (sizeof(T) == 8) {
       rc = launch_ring_anal_f64(p, (const double *)src, pixw, wc, (double *)F, s);
       if (rc) return rc;
       rc = launch_legendre_anal_f64(p, (const double *)F, (double *)alm, (double *)partial, it > 0,
                                     s);
     } else {
-      rc = launch_ring_anal_f32(p, S, (const float *)src, (float *)F, s);
+      rc = launch_ring_anal_f32(p, S, (const float *)src, pixw, wc, (float *)F, s);
+      if (pixw && rc == GA_ERR_UNSUPPORTED) {  // weights in a pass of their own
+        clear_error();
+        hipLaunchKernelGGL(weight_pixels_kernel, dim3(unsigned((npx + 255) / 256)), dim3(256), 0,
+                           s, npx, int64_t(p->npix), (const float *)src, pixw, wc,
+                           (float *)map_tmp);
+        GA_LAUNCH_CHECK();
+        rc = launch_ring_anal_f32(p, S, (const float *)map_tmp, nullptr, 0.0, (float *)F, s);
+      }
       if (rc) return rc;
       rc = launch_legendre_anal_f32(p, S, (const float *)F, (float *)alm, (float *)partial, it > 0,
                                     s);

@@ -73,7 +73,10 @@ int launch_ring_synth_f32(const ga_plan *p, int S, int G, const float *F, float 
 // (FP64: one map; with pixw, pixel p is first multiplied by pixw[p] wc)
 int launch_ring_anal_f64(const ga_plan *p, const double *maps, const double *pixw, double wc,
                          double *F, hipStream_t s);
-int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, float *F, hipStream_t s);
+// FP32: with pixw, pixel p of every map is first multiplied by pixw[p] wc
+// (register form only: GA_ERR_UNSUPPORTED with nothing launched otherwise)
+int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, const double *pixw,
+                         double wc, float *F, hipStream_t s);
 // out = ref - FP32 ring synthesis of F (fused-pass forms only; GA_ERR_UNSUPPORTED
 // with nothing launched otherwise)
 int launch_ring_resid_f32(const ga_plan *p, int S, int G, const float *F, float *out,

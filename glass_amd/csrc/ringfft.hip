@@ -1455,7 +1455,10 @@ int launch_blu_class(const ga_plan *p, const int32_t *list, int nlist, int max_r
 // The two real transforms are split with the partner bin n - k, exchanged
 // through LDS in two halves (bins k2 = 2, 3 first, for the outputs of
 // k2 = 0, 1; then the other way), and every m = k (mod n), m <= lmax, gets
-// weight e^{-i m phi0} (d0, d1) stored as one 16-byte pair.
+// weight e^{-i m phi0} (d0, d1) stored as one 16-byte pair.  pixw: pixel p is
+// multiplied by pixw[p] wc in the load, in FP64 and rounded once, as the pass
+// of its own did that this saves (64 maps at nside 1024: 2.1 ms, of which 0.4 come back
+// here).
 template <int NT, int C, bool BLU>
 __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_kernel(
     int lmax, const int32_t *__restrict__ ring_list, int nlist,
@@ -1463,7 +1466,8 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
     const int32_t *__restrict__ ring_pnum, const int32_t *__restrict__ ring_pden,
     const int64_t *__restrict__ blu_off, const float2 *__restrict__ blu,
     const float2 *__restrict__ tw, int twlen, int ldx, const float *__restrict__ maps, int S,
-    int nunit, int64_t npix, float weight, cplx<float> *__restrict__ F) {
+    int nunit, int64_t npix, float weight, cplx<float> *__restrict__ F,
+    const double *__restrict__ pixw, double wc) {
   extern __shared__ char smem_raw[];
   cplx<float> *X = reinterpret_cast<cplx<float> *>(smem_raw);
   int li, unit;
@@ -1489,6 +1493,16 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
     if (j1 < r) {
       a = reinterpret_cast<const float4 *>(maps + int64_t(s0) * npix + st)[j1];
       if (two) b = reinterpret_cast<const float4 *>(maps + int64_t(s0 + 1) * npix + st)[j1];
+    }
+    if (pixw && j1 < r) {
+      // the quadrature weights of the ring's pixels, the same for every shell
+      // (all units of a ring run on one XCD: its L2 serves them after the first)
+      const double *__restrict__ pw = pixw + st + 4 * j1;
+      const double w0 = pw[0] * wc, w1 = pw[1] * wc, w2 = pw[2] * wc, w3 = pw[3] * wc;
+      a = float4{float(double(a.x) * w0), float(double(a.y) * w1), float(double(a.z) * w2),
+                 float(double(a.w) * w3)};
+      b = float4{float(double(b.x) * w0), float(double(b.y) * w1), float(double(b.z) * w2),
+                 float(double(b.w) * w3)};
     }
     x[c][0] = cplx<float>{a.x, b.x};
     x[c][1] = cplx<float>{a.y, b.y};
@@ -1621,7 +1635,7 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
 
 template <int NT, int C, bool BLU>
 int launch_anal2(const ga_plan *p, const int32_t *list, int nlist, int maxN, int S,
-                 const float *maps, float *F, hipStream_t stream) {
+                 const float *maps, const double *pixw, double wc, float *F, hipStream_t stream) {
   if (nlist == 0) return GA_OK;
   const int ldx = padded_len(maxN);
   const size_t lds = size_t(2) * ldx * sizeof(cplx<float>);
@@ -1634,15 +1648,16 @@ int launch_anal2(const ga_plan *p, const int32_t *list, int nlist, int maxN, int
   hipLaunchKernelGGL(kfn, dim3(unsigned(nblk)), dim3(NT), lds, stream, p->lmax, list, nlist,
                      p->d_ring_start, p->d_ring_n, p->d_ring_pnum, p->d_ring_pden, p->d_blu_off,
                      p->d_blu32, p->d_tw32, p->tw_len, ldx, maps, S, nunit, p->npix,
-                     float(4.0 * M_PI / double(p->npix)), reinterpret_cast<cplx<float> *>(F));
+                     float(4.0 * M_PI / double(p->npix)), reinterpret_cast<cplx<float> *>(F), pixw,
+                     wc);
   GA_LAUNCH_CHECK();
   return GA_OK;
 }
 
 // both ring classes by the register form; GA_ERR_UNSUPPORTED (before any
 // launch) outside its sizes or alignment
-int launch_ring_anal2_f32(const ga_plan *p, int S, const float *maps, float *F,
-                          hipStream_t stream) {
+int launch_ring_anal2_f32(const ga_plan *p, int S, const float *maps, const double *pixw,
+                          double wc, float *F, hipStream_t stream) {
   if (reinterpret_cast<uintptr_t>(maps) & 15) return GA_ERR_UNSUPPORTED;
   if (S > 1 && (reinterpret_cast<uintptr_t>(F) & 15)) return GA_ERR_UNSUPPORTED;
   const int rp = p->max_r_pow2, rb = p->max_r_blu, Lb = p->max_L_blu;
@@ -1652,20 +1667,20 @@ int launch_ring_anal2_f32(const ga_plan *p, int S, const float *maps, float *F,
   if (p->n_pow2 > 0) {
     const int32_t *l = p->d_rings_pow2;
     const int n = p->n_pow2;
-    if (rp <= 256) rc = launch_anal2<256, 1, false>(p, l, n, rp, S, maps, F, stream);
-    else if (rp <= 512) rc = launch_anal2<256, 2, false>(p, l, n, rp, S, maps, F, stream);
-    else if (rp <= 1024) rc = launch_anal2<256, 4, false>(p, l, n, rp, S, maps, F, stream);
-    else if (rp <= 2048) rc = launch_anal2<256, 8, false>(p, l, n, rp, S, maps, F, stream);
-    else rc = launch_anal2<512, 8, false>(p, l, n, rp, S, maps, F, stream);
+    if (rp <= 256) rc = launch_anal2<256, 1, false>(p, l, n, rp, S, maps, pixw, wc, F, stream);
+    else if (rp <= 512) rc = launch_anal2<256, 2, false>(p, l, n, rp, S, maps, pixw, wc, F, stream);
+    else if (rp <= 1024) rc = launch_anal2<256, 4, false>(p, l, n, rp, S, maps, pixw, wc, F, stream);
+    else if (rp <= 2048) rc = launch_anal2<256, 8, false>(p, l, n, rp, S, maps, pixw, wc, F, stream);
+    else rc = launch_anal2<512, 8, false>(p, l, n, rp, S, maps, pixw, wc, F, stream);
     if (rc) return rc;
   }
   if (p->n_blu > 0) {
     const int32_t *l = p->d_rings_blu;
     const int n = p->n_blu;
-    if (rb <= 256) rc = launch_anal2<256, 1, true>(p, l, n, Lb, S, maps, F, stream);
-    else if (rb <= 512) rc = launch_anal2<256, 2, true>(p, l, n, Lb, S, maps, F, stream);
-    else if (rb <= 1024) rc = launch_anal2<256, 4, true>(p, l, n, Lb, S, maps, F, stream);
-    else rc = launch_anal2<512, 4, true>(p, l, n, Lb, S, maps, F, stream);
+    if (rb <= 256) rc = launch_anal2<256, 1, true>(p, l, n, Lb, S, maps, pixw, wc, F, stream);
+    else if (rb <= 512) rc = launch_anal2<256, 2, true>(p, l, n, Lb, S, maps, pixw, wc, F, stream);
+    else if (rb <= 1024) rc = launch_anal2<256, 4, true>(p, l, n, Lb, S, maps, pixw, wc, F, stream);
+    else rc = launch_anal2<512, 4, true>(p, l, n, Lb, S, maps, pixw, wc, F, stream);
   }
   return rc;
 }
@@ -1842,12 +1857,14 @@ int launch_ring_resid_f32(const ga_plan *p, int S, int G, const float *F, float 
   if (rc == GA_ERR_UNSUPPORTED) clear_error();
   return rc;
 }
-int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, float *F, hipStream_t s) {
+int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, const double *pixw,
+                         double wc, float *F, hipStream_t s) {
   if (p->tune.ring_path != 1) {
-    const int rc = launch_ring_anal2_f32(p, S, maps, F, s);
+    const int rc = launch_ring_anal2_f32(p, S, maps, pixw, wc, F, s);
     if (rc != GA_ERR_UNSUPPORTED) return rc;
     clear_error();
   }
+  if (pixw) return GA_ERR_UNSUPPORTED;  // the first form does not weight
   return launch_ring<float>(p, S, S, maps, F, nullptr, true, s);
 }
 

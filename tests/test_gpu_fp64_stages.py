@@ -157,3 +157,34 @@ def test_alm_order(nl):
     _lib.call("ga_glass_to_healpix_alm_f64", nl, _lib.ptr(a), _lib.ptr(out), _lib.stream_ptr())
     ref = np.concatenate([np.arange(m, nl) * (np.arange(m, nl) + 1) // 2 + m for m in range(nl)])
     np.testing.assert_array_equal(out.cpu().numpy().real, ref)
+
+
+@pytest.mark.parametrize("S,offset,path", [(1, 0, 0), (3, 0, 0), (4, 1, 0), (5, 2, 0), (3, 0, 1)])
+def test_weighted_batch_analysis_routes(S, offset, path):
+    """Weights in the ring stage's load (16-byte aligned maps, register form) and
+    in a pass of their own (maps off by one or two floats; the first ring form)
+    against the FP64 analysis of the same maps."""
+    nside, lmax, niter = 24, 48, 1
+    npix = 12 * nside * nside
+    rng = np.random.default_rng(S + offset)
+    maps = rng.standard_normal((S, npix)).astype(np.float32)
+    buf = torch.empty(S * npix + 4, dtype=torch.float32, device="cuda")
+    d = buf[offset:offset + S * npix]
+    d.copy_(torch.as_tensor(maps.reshape(-1)))
+    w = hp.pixel_weights(nside)
+    plan = _lib.get_plan(nside, lmax)
+    plan.set_tuning(_lib.TUNE_RING_PATH, path)
+    try:
+        ws = _lib.workspace(plan.workspace_bytes(S, 4, analysis=True))
+        tmp = torch.empty(S * npix, dtype=torch.float32, device="cuda")
+        alm = torch.empty((O.nalm(lmax), S), dtype=torch.complex64, device="cuda")
+        _lib.call("ga_map2alm_weighted_batch_f32", plan.h, S, _lib.ptr(d), _lib.ptr(w),
+                  _lib.ptr(alm), niter, _lib.ptr(tmp), _lib.ptr(ws), ws.numel(),
+                  _lib.stream_ptr())
+    finally:
+        plan.set_tuning(_lib.TUNE_RING_PATH, 0)
+    got = alm.cpu().numpy()
+    for s in range(S):
+        ref = O.map2alm_weighted(maps[s].astype(np.float64), w.cpu().numpy(), lmax, niter)
+        err = np.max(np.abs(got[:, s] - ref)) / np.sqrt(np.mean(np.abs(ref) ** 2))
+        assert err < 1e-5  # the FP32 path's target, as in the other tests
