@@ -37,7 +37,7 @@ using f16::split_pair;
 constexpr int kAWaves = 8;                // waves per workgroup
 constexpr int kAPairs = 64 * kAWaves;     // ring pairs per workgroup = one partial slot
 constexpr int kASlab = 64;                // l rows per slab
-constexpr int kARowPad = 8;               // halves of padding per LDS row of lambda
+constexpr int kARowPad = 4;               // words of padding per LDS row of lambda
 constexpr int kAColTop = 13;              // column maxima are scaled below 2^13
 
 __device__ __forceinline__ int anal_shift(float mx) {
@@ -45,6 +45,20 @@ __device__ __forceinline__ int anal_shift(float mx) {
   int e;
   (void)frexpf(mx, &e);  // mx < 2^e
   return kAColTop - e;
+}
+
+// x = hi + lo in one word, hi (rounded toward zero) in the low half, the
+// residual rounded to nearest in the high half: the values of split_pair
+__device__ __forceinline__ uint32_t split_word(float x) {
+  uint32_t r = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, 0.0f));
+  asm("v_fma_mixhi_f16 %0, %1, 1.0, -%0 op_sel_hi:[0,0,1]" : "+v"(r) : "v"(x));
+  return r;
+}
+__device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x05040100u);
+}
+__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
 template <int NT>
@@ -126,16 +140,18 @@ __global__ __launch_bounds__(64 * kAWaves, 1) void legendre_anal_f16_kernel(
     __builtin_amdgcn_sched_barrier(0);  // one tile's raw values live at a time
   }
 
-  // LDS: per wave the transposed slab lam[hi|lo][parity][l' (32)][pair (64)],
-  // rows padded by 8 halves (16 bytes) so that the 16-byte A reads of 8
-  // consecutive lanes (rows 144 bytes apart) fall in distinct banks (18 KB);
+  // LDS: per wave the transposed slab lam[parity][l' (32)][pair (64)], each
+  // value as its two FP16 halves in one word (a 16-bit store costs the LDS as
+  // much as a 32-bit one: the two halves in arrays of their own took twice the
+  // stores; 7.85 -> 7.55 ms per analysis of 64 maps at nside 1024, lmax 2047), rows padded by 4 words so that the 16-byte A reads of 16
+  // consecutive lanes (rows 272 bytes apart) fall in distinct banks (17 KB);
   // after the MFMAs of a slab the same memory holds the waves' D tiles for
   // the fixed-order sum.  Recurrence coefficients gam_l are the same for
   // every wave of the workgroup (one m): one double buffer of one slab,
   // written by wave 0, read after the slab's barriers.
-  __shared__ __align__(16) _Float16 lam[kAWaves][2][2][32][64 + kARowPad];
+  __shared__ __align__(16) uint32_t lam[kAWaves][2][32][64 + kARowPad];
   __shared__ double cbuf[2][kASlab];
-  float *red = reinterpret_cast<float *>(&lam[0][0][0][0][0]);  // [wave][p][e][lane]
+  float *red = reinterpret_cast<float *>(&lam[0][0][0][0]);  // [wave][p][e][lane]
 
   const int64_t base = hp_index(lmax, m, m);
   const double *__restrict__ co = gam + base;
@@ -143,7 +159,7 @@ __global__ __launch_bounds__(64 * kAWaves, 1) void legendre_anal_f16_kernel(
   double cpre = co[min(lane, lastc)];
   if (wave == 0) cbuf[0][lane] = cpre;
   __syncthreads();
-  _Float16(*lw)[2][32][64 + kARowPad] = lam[wave];  // [hi|lo][p][l'][pair]
+  uint32_t(*lw)[32][64 + kARowPad] = lam[wave];  // [p][l'][pair]
 
   const int nsl = (lmax - m + kASlab) / kASlab;
   // Leading slabs in which every lane of the workgroup either starts scaled
@@ -233,19 +249,11 @@ __global__ __launch_bounds__(64 * kAWaves, 1) void legendre_anal_f16_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = float(d[j]);
       }
-      uint32_t h0, l0w, h1, l1w;
-      split_pair(v[0], v[2], h0, l0w);  // parity 0, rows 2g, 2g + 1
-      split_pair(v[1], v[3], h1, l1w);  // parity 1
-      const f16::f16x2 H0 = __builtin_bit_cast(f16::f16x2, h0), L0 = __builtin_bit_cast(f16::f16x2, l0w);
-      const f16::f16x2 H1 = __builtin_bit_cast(f16::f16x2, h1), L1 = __builtin_bit_cast(f16::f16x2, l1w);
-      lw[0][0][2 * g][lane] = H0[0];
-      lw[0][0][2 * g + 1][lane] = H0[1];
-      lw[1][0][2 * g][lane] = L0[0];
-      lw[1][0][2 * g + 1][lane] = L0[1];
-      lw[0][1][2 * g][lane] = H1[0];
-      lw[0][1][2 * g + 1][lane] = H1[1];
-      lw[1][1][2 * g][lane] = L1[0];
-      lw[1][1][2 * g + 1][lane] = L1[1];
+      // parity 0: rows 2g, 2g + 1; parity 1: the same
+      lw[0][2 * g][lane] = split_word(v[0]);
+      lw[1][2 * g][lane] = split_word(v[1]);
+      lw[0][2 * g + 1][lane] = split_word(v[2]);
+      lw[1][2 * g + 1][lane] = split_word(v[3]);
     }
     if (wave == 0) cbuf[cur ^ 1][lane] = cpre;  // read after this slab's barriers
 
@@ -258,8 +266,14 @@ __global__ __launch_bounds__(64 * kAWaves, 1) void legendre_anal_f16_kernel(
     for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        const f16x8 ah = *reinterpret_cast<const f16x8 *>(&lw[0][p][c32][16 * kb + 8 * half]);
-        const f16x8 al = *reinterpret_cast<const f16x8 *>(&lw[1][p][c32][16 * kb + 8 * half]);
+        const uint4 *aw = reinterpret_cast<const uint4 *>(&lw[p][c32][16 * kb + 8 * half]);
+        const uint4 w0 = aw[0], w1 = aw[1];
+        const f16x8 ah = __builtin_bit_cast(
+            f16x8, uint4{low_halves(w0.x, w0.y), low_halves(w0.z, w0.w), low_halves(w1.x, w1.y),
+                         low_halves(w1.z, w1.w)});
+        const f16x8 al = __builtin_bit_cast(
+            f16x8, uint4{high_halves(w0.x, w0.y), high_halves(w0.z, w0.w),
+                         high_halves(w1.x, w1.y), high_halves(w1.z, w1.w)});
 #pragma unroll
         for (int ct = 0; ct < NT; ++ct) {
           const f16x8 Bh = __builtin_bit_cast(f16x8, bh[ct][p][kb]);
