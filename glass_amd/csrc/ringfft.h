@@ -41,12 +41,12 @@ __host__ __device__ inline int padded_len(int n) {
   return n + (n >> kPadShift<T>) + 1;
 }
 
-__device__ __forceinline__ cplx<float> expi_q(int64_t q, int64_t d, float) {
+__device__ __forceinline__ cplx<float> expi_q(int q, int d, float) {
   float s, c;
   sincospif(2.0f * float(q) / float(d), &s, &c);
   return {c, s};
 }
-__device__ __forceinline__ cplx<double> expi_q(int64_t q, int64_t d, double) {
+__device__ __forceinline__ cplx<double> expi_q(int q, int d, double) {
   double s, c;
   sincospi(2.0 * double(q) / double(d), &s, &c);
   return {c, s};

@@ -1562,11 +1562,23 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
     __syncthreads();
   }
 
+  // j / n to one rounding without the division (exact for a power of two)
+  const float fn = float(n), inv = 1.0f / fn;
+  auto over_n = [&](int j) {
+    const float v = float(j), q0 = v * inv;
+    return fmaf(fmaf(-q0, fn, v), inv, q0);
+  };
+  auto expi_neg = [](float u) {  // e^{-i pi u}
+    float s, c;
+    sincospif(u, &s, &c);
+    return cplx<float>{c, -s};
+  };
+
   // ---- radix-4 combination: bins k1 + r k2 into x[c][k2]
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     const int k1 = min(t + c * NT, r - 1);
-    const cplx<float> w1 = cconj(expi_q(k1, n, 0.0f));
+    const cplx<float> w1 = expi_neg(2.0f * over_n(k1));
     const cplx<float> w2 = cmul(w1, w1), w3 = cmul(w2, w1);
     const cplx<float> y0 = x[c][0], y1 = cmul(x[c][1], w1), y2 = cmul(x[c][2], w2),
                       y3 = cmul(x[c][3], w3);
@@ -1584,6 +1596,7 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
   cplx<float> *Fr = F + int64_t(ring) * (lmax + 1) * S + s0;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
+    if (h == 1 && 2 * r > lmax) break;  // no bin of the second half has an m
     // LDS holds the other half: bins k2 = 2 - 2h + a at X[a ldx + pad(k1)]
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -1610,13 +1623,13 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
         const cplx<float> av = xv, bv = cconj(pv);
         const cplx<float> d0 = {0.5f * (av.re + bv.re), 0.5f * (av.im + bv.im)};
         const cplx<float> d1 = {0.5f * (av.im - bv.im), -0.5f * (av.re - bv.re)};  // (a - b) / (2i)
-        // ring phase e^{-i m phi0}, m phi0 = 2 pi (m pnum mod pden) / pden, stepped by n
-        int q = pnum ? int(int64_t(k) * pnum % pden) : 0;
-        const int dq = pnum ? int(int64_t(n) * pnum % pden) : 0;
+        // ring phase e^{-i m phi0}, m phi0 = pi (m mod 2 n) / n, stepped by n
+        // (phi0 is 0 or pi / n: pnum is 0 or 1, pden is 2 n)
+        int q = k;
         for (int mm = k; mm <= lmax; mm += n) {
-          const cplx<float> ph = pnum ? cconj(expi_q(q, pden, 0.0f)) : cplx<float>{1.0f, 0.0f};
-          q += dq;
-          if (q >= pden) q -= pden;
+          const cplx<float> ph = pnum ? expi_neg(over_n(q)) : cplx<float>{1.0f, 0.0f};
+          q += n;
+          if (q >= 2 * n) q -= 2 * n;
           const cplx<float> v0 = cmul(d0, ph), v1 = cmul(d1, ph);
           cplx<float> *f = Fr + int64_t(mm) * S;
           if (two && !(S & 1)) {  // the pair is 16-byte aligned
