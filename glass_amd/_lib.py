@@ -184,7 +184,11 @@ def require_gpu() -> None:
 
 
 def stream_ptr():
-    return ctypes.c_void_p(torch().cuda.current_stream().cuda_stream)
+    # the current stream's handle without a torch Stream object around it: 0.5
+    # us against 2.9, paid once per launch (alm2map at nside 32: 18.4 -> 15.7
+    # us; generate, 10 shells at nside 128: 985 -> 904 us)
+    t = torch()
+    return ctypes.c_void_p(t._C._cuda_getCurrentRawStream(t.cuda.current_device()))
 
 
 def ptr(t) -> ctypes.c_void_p:
