@@ -595,7 +595,8 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[2][2][NT], int m,
 // SEP: the two-chunk form parks in a region of its own (park_lanes) instead
 // of in F (park_tile); one variant per kernel keeps the register allocation
 // of each within the 256 registers of two waves per SIMD.
-template <int NT, bool FLUSH, bool SEP>
+// NT column tiles per wave of the TB that each column group of the grid has.
+template <int NT, bool FLUSH, bool SEP, int TB = NT>
 __device__ __forceinline__ void contract_blocks(const f16_geom &g, const int b) {
   const int lmax = g.lmax, npairs = g.npairs, nrings = g.nrings, ncols = g.ncols, nct = g.nct,
             nrg = g.nrg, ncg = g.ncg, lam_exp = g.lam_exp, flush = g.flush, nchunk = g.nchunk;
@@ -648,11 +649,11 @@ __device__ __forceinline__ void contract_blocks(const f16_geom &g, const int b) 
   const int64_t s0 = slab_off[m];
   const int nsl = int(nslab_of(lmax, m));
   const int half = lane >> 5, col_in = lane & 31;
-  const int colbase = cg * 32 * NT;
+  const int colbase = cg * 32 * TB;
   // column tiles past the last real one re-read the last tile (never stored)
   int ctile[NT];
 #pragma unroll
-  for (int ct = 0; ct < NT; ++ct) ctile[ct] = min(cg * NT + ct, nct - 1);
+  for (int ct = 0; ct < NT; ++ct) ctile[ct] = min(cg * TB + ct, nct - 1);
 
   f32x16 acc[2][2][NT];  // [parity][row tile][col tile]
   f32x16 mst[2][2][FLUSH ? NT : 1];  // master sums of the flushing form
@@ -745,7 +746,7 @@ __device__ __forceinline__ void contract_blocks(const f16_geom &g, const int b) 
   const bool two = !FLUSH && nchunk == 2 && nsl - s >= g.chunk_min;
   run_slabs(two ? s + (nsl - s) / 2 : nsl);
   if (two) {
-    if (SEP) park_lanes<NT, false>(acc, g.part + park_slot(m, rem, G, wave, NT) + lane);
+    if (SEP) park_lanes<NT, false>(acc, g.part + park_slot(m, rem, G, wave, TB) + lane);
     else park_tile<NT, false>(acc, m, lmax, npairs, nrings, ncols, colbase, rp0, lane, F, eqo, g.cshift);
 #pragma unroll
     for (int p = 0; p < 2; ++p)
@@ -754,7 +755,7 @@ __device__ __forceinline__ void contract_blocks(const f16_geom &g, const int b) 
 #pragma unroll
         for (int ct = 0; ct < NT; ++ct) acc[p][t][ct] = f32x16{};
     run_slabs(nsl);
-    if (SEP) park_lanes<NT, true>(acc, g.part + park_slot(m, rem, G, wave, NT) + lane);
+    if (SEP) park_lanes<NT, true>(acc, g.part + park_slot(m, rem, G, wave, TB) + lane);
     else park_tile<NT, true>(acc, m, lmax, npairs, nrings, ncols, colbase, rp0, lane, F, eqo, g.cshift);
   }
   if (FLUSH) {
@@ -772,6 +773,21 @@ __device__ __forceinline__ void contract_blocks(const f16_geom &g, const int b) 
 template <int NT, int MINW, bool FLUSH, bool SEP>
 __global__ __launch_bounds__(256, MINW) void legendre_synth_f16_kernel(const f16_geom g) {
   contract_blocks<NT, FLUSH, SEP>(g, int(blockIdx.x));
+}
+
+// Two tiles per wave, an odd number of them: the last column group has one,
+// and its waves run the one-tile body instead of computing that tile twice
+// (bit-identical; 40 shells at nside 1024, lmax 2047: 6.3 -> 5.9 ms for the
+// whole batch; 33 shells at nside 512, lmax 1023: 1254 -> 1242 us).  A kernel
+// of its own: the two bodies are 68 KB of code, more than the instruction
+// cache, which an even number of tiles need not carry.
+template <bool SEP>
+__global__ __launch_bounds__(256, 2) void legendre_synth_f16_odd_kernel(const f16_geom g) {
+  const int b = int(blockIdx.x);
+  if ((b >> 3) % g.ncg == g.ncg - 1)
+    contract_blocks<1, false, SEP, 2>(g, b);
+  else
+    contract_blocks<2, false, SEP>(g, b);
 }
 
 // Several geometries in one grid (an uneven batch): geometry i owns blocks
@@ -1076,6 +1092,12 @@ int launch_legendre_contract_f16(const ga_plan *p, int S, float *F, const void *
   if (flush > 0) GA_F16_LAUNCH(1, 2, true, false);
   else if (nt == 1 && flush == -3) GA_F16_LAUNCH(1, 2, false, true);
   else if (nt == 1) GA_F16_LAUNCH(1, 2, false, false);
+  else if (nct % 2 && flush == -3)
+    hipLaunchKernelGGL(legendre_synth_f16_odd_kernel<true>, dim3(unsigned(nblk2)), dim3(256), 0,
+                       stream, g);
+  else if (nct % 2)
+    hipLaunchKernelGGL(legendre_synth_f16_odd_kernel<false>, dim3(unsigned(nblk2)), dim3(256), 0,
+                       stream, g);
   else if (flush == -3) GA_F16_LAUNCH(2, 2, false, true);
   else GA_F16_LAUNCH(2, 2, false, false);
 #undef GA_F16_LAUNCH
