@@ -160,9 +160,9 @@ int launch_legendre_synth_f64(const ga_plan *p, const double *alm, double *F, do
   // The normalised form saves an operation in five and, with two pairs per
   // lane, half the scalar loads, but costs the launch of the scaling pass and
   // the wait between the two, and half the waves.  Measured (whole alm2map):
-  // nside 256, lmax 512 (4104 waves of one pair per lane): plain 53.6 us,
-  // normalised 76; nside 512, lmax 1023 (16384 waves): 222 and 209 us; nside
-  // 1024, lmax 2048: 1232 and 1003 us.
+  // nside 256, lmax 512 (4104 waves of one pair per lane): plain 34 us,
+  // normalised 69; nside 512, lmax 1023 (16384 waves): 142 and 133 us; nside
+  // 1024, lmax 2048: 991 and 763 us.
   const int64_t waves = int64_t(p->lmax + 1) * ((p->npairs + 63) / 64);
   if (waves < kManyWaves || scratch_doubles < size_t(2 * p->nalm))
     return launch<1, false>(p, alm, F, stream);
