@@ -1459,11 +1459,16 @@ int launch_blu_class(const ga_plan *p, const int32_t *list, int nlist, int max_r
 // multiplied by pixw[p] wc in the load, in FP64 and rounded once, as the pass
 // of its own did that this saves (64 maps at nside 1024: 2.1 ms, of which 0.4 come back
 // here).
+//
+// Bound: the unfolding as much as the transforms.  64 maps at nside 1024, lmax
+// 2047: power-of-two rings 2.28 ms, Bluestein rings 2.49 ms (2.39 and 2.65 with
+// 64-bit remainders and divisions in the ring phases); without the unfolding
+// 1.02 and 1.86, without the transforms 2.31 and 1.59.
 template <int NT, int C, bool BLU>
 __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_kernel(
     int lmax, const int32_t *__restrict__ ring_list, int nlist,
     const int64_t *__restrict__ ring_start, const int32_t *__restrict__ ring_n,
-    const int32_t *__restrict__ ring_pnum, const int32_t *__restrict__ ring_pden,
+    const int32_t *__restrict__ ring_pnum,
     const int64_t *__restrict__ blu_off, const float2 *__restrict__ blu,
     const float2 *__restrict__ tw, int twlen, int ldx, const float *__restrict__ maps, int S,
     int nunit, int64_t npix, float weight, cplx<float> *__restrict__ F,
@@ -1477,7 +1482,7 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
   const int s0 = 2 * unit;
   const bool two = s0 + 1 < S;
   const int n = ring_n[ring], r = n >> 2;
-  const int pnum = ring_pnum[ring], pden = ring_pden[ring];
+  const int pnum = ring_pnum[ring];
   const int64_t st = ring_start[ring];
   const float2 *__restrict__ chirp = BLU ? blu + blu_off[r] : blu;
   const float2 *__restrict__ bspec = chirp + r;
@@ -1624,7 +1629,7 @@ __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_
         const cplx<float> d0 = {0.5f * (av.re + bv.re), 0.5f * (av.im + bv.im)};
         const cplx<float> d1 = {0.5f * (av.im - bv.im), -0.5f * (av.re - bv.re)};  // (a - b) / (2i)
         // ring phase e^{-i m phi0}, m phi0 = pi (m mod 2 n) / n, stepped by n
-        // (phi0 is 0 or pi / n: pnum is 0 or 1, pden is 2 n)
+        // (phi0 is 0 or pi / n: pnum is 0 or 1)
         int q = k;
         for (int mm = k; mm <= lmax; mm += n) {
           const cplx<float> ph = pnum ? expi_neg(over_n(q)) : cplx<float>{1.0f, 0.0f};
@@ -1659,8 +1664,8 @@ int launch_anal2(const ga_plan *p, const int32_t *list, int nlist, int maxN, int
   GA_CHECK_HIP(hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    int(lds)));
   hipLaunchKernelGGL(kfn, dim3(unsigned(nblk)), dim3(NT), lds, stream, p->lmax, list, nlist,
-                     p->d_ring_start, p->d_ring_n, p->d_ring_pnum, p->d_ring_pden, p->d_blu_off,
-                     p->d_blu32, p->d_tw32, p->tw_len, ldx, maps, S, nunit, p->npix,
+                     p->d_ring_start, p->d_ring_n, p->d_ring_pnum, p->d_blu_off, p->d_blu32,
+                     p->d_tw32, p->tw_len, ldx, maps, S, nunit, p->npix,
                      float(4.0 * M_PI / double(p->npix)), reinterpret_cast<cplx<float> *>(F), pixw,
                      wc);
   GA_LAUNCH_CHECK();
