@@ -15,7 +15,9 @@
 // time.  Values far below the range that matters are kept scaled
 // (to_scaled_low) and rescaled once per chunk, so no step has a test.  Skipping
 // the sums while a whole wave is scaled would save 1 to 5 % (nside 300, 1024),
-// but a coefficient that is not finite would then not reach every ring.
+// but a coefficient that is not finite would then not reach every ring.  The
+// coefficients below the spin (l < s, which a spin-s field does not have) never
+// enter a sum, whatever they hold.
 //
 // Bound: FP64 issue, 14 operations per (l, m, ring pair).  Measured at nside
 // 300, lmax 767 (E and B): 141 us (chunks of 4 rows 169 us, two ring pairs per
@@ -113,7 +115,8 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
   const double *__restrict__ cf = tab + 3 * base;
   const double2 *__restrict__ e = E + base, *__restrict__ b = B + base;
   const int nl = lmax + 1 - m;
-  int i = (l0 - m) & ~1;
+  const int first = l0 - m;  // the first row of the sums
+  int i = first & ~1;
   bool scaled = s.any_scaled();  // wave-uniform
   for (; i + kChunk <= nl; i += kChunk) {
     double c[3 * kChunk];
@@ -124,6 +127,7 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
     for (int q = 0; q < kChunk; ++q) ev[q] = e[i + q];
 #pragma unroll
     for (int q = 0; q < kChunk; ++q) bv[q] = b[i + q];
+    if (i < first) ev[0] = bv[0] = double2{0.0, 0.0};  // l = l0 - 1, below the spin
 #pragma unroll
     for (int q = 0; q < kChunk; ++q) {
       s.advance(c[3 * q], c[3 * q + 1], c[3 * q + 2]);
@@ -138,7 +142,8 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
   for (int q = 0; q < kChunk - 1; ++q)  // the last rows (the chunks leave i even)
     if (i + q < nl) {
       s.advance(cf[3 * (i + q)], cf[3 * (i + q) + 1], cf[3 * (i + q) + 2]);
-      s.add(q & 1, e[i + q], b[i + q]);
+      const bool below = q == 0 && i < first;
+      s.add(q & 1, below ? double2{0.0, 0.0} : e[i + q], below ? double2{0.0, 0.0} : b[i + q]);
     }
 
   const double sg = (spin & 1) ? -1.0 : 1.0;
