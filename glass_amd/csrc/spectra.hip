@@ -84,7 +84,7 @@ __global__ __launch_bounds__(64) void cl2corr_kernel(int nl, const double *__res
   const double xk = x[min(k, n - 1)];
   auto fill = [&](int buf, int l0) {
     const int l = l0 + lane;
-    ab[buf][lane] = legendre_row(l);
+    ab[buf][lane] = l < nl ? legendre_row(l) : double2{0.0, 0.0};
     c[buf][lane] = l < nl ? cl[l] * (double(2 * l + 1) / (4.0 * M_PI)) : 0.0;
   };
   double p0 = 1.0, p1 = 0.0, acc = 0.0;
@@ -94,7 +94,9 @@ __global__ __launch_bounds__(64) void cl2corr_kernel(int nl, const double *__res
   for (int l0 = 0; l0 < nl; l0 += 64, buf ^= 1) {
     if (l0 + 64 < nl) fill(buf ^ 1, l0 + 64);
     // 16 rows to registers while the 16 before them are run: a wave that is
-    // alone on its CU hides no latency; rows past nl have c = 0
+    // alone on its CU hides no latency; rows past nl have c = 0 and values of
+    // zero (a node with |x| > 1, where P_l grows without bound, must not
+    // overflow in them)
     double2 r[4][16];
     double cv[4][16];
 #pragma unroll
