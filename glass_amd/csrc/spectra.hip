@@ -8,12 +8,11 @@
 //
 // With n Gauss-Legendre nodes (x_k, w_k) and n coefficients l < n the pair is
 // exact (products P_l P_l' of degree < 2n - 1 are integrated exactly), so
-// corr2cl(cl2corr(cl)) = cl to rounding.  P_l by its three-term recurrence in
-// FP64, one lane per node; corr2cl reduces 32 l at a time over the 64 nodes of
-// a wave and then over waves in a fixed order, so the result does not depend
-// on scheduling.  The nodes come from Newton's method on P_n
-// from the asymptotic first guess cos(pi (i + 3/4) / (n + 1/2)), one thread
-// per node pair (x, -x).
+// corr2cl(cl2corr(cl)) = cl to rounding.  P_l by a recurrence in l in FP64, one
+// lane per node; corr2cl reduces 32 l at a time over the 64 nodes of a wave and
+// then over waves in a fixed order, so the result does not depend on scheduling.
+// The nodes come from Newton's method on P_n from the asymptotic first guess
+// cos(pi (i + 3/4) / (n + 1/2)), one thread per node pair (x, -x).
 #include "common.h"
 #include "device.h"
 #include "kernels.h"
@@ -57,54 +56,62 @@ __global__ __launch_bounds__(256) void gl_nodes_kernel(int n, double *__restrict
   if ((n & 1) && i == n / 2) x[i] = 0.0;
 }
 
-// Rows of the recurrence P_l = (a_l x) P_{l-1} - b_l P_{l-2}, a_l = (2l-1)/l, b_l =
-// (l-1)/l, for kChunk values of l at a time: lane i works out row l0 + i (its
-// divisions would otherwise be done by every lane in every step) into LDS,
-// from where all lanes read it; the row of l = 0, (0, -1), yields P_0 = 1 from
-// (P_{-2}, P_{-1}) = (1, 0).
-__device__ __forceinline__ double2 legendre_row(int l) {
-  return l == 0 ? double2{0.0, -1.0} : double2{double(2 * l - 1) / l, double(l - 1) / l};
-}
-__device__ __forceinline__ double legendre_step(double2 ab, double x, double &p0, double &p1) {
-  const double p = fma(ab.x * x, p1, -(ab.y * p0));
-  p0 = p1;
-  p1 = p;
+// P_l by differences: with D_l = P_l - P_{l-1} and s = 1 / l,
+//   D_l = (1 - s) D_{l-1} + (2 - s) (x - 1) P_{l-1},   P_l = P_{l-1} + D_l.
+// Near x = 1, where the three-term form loses most (its coefficients tend to the
+// constants 2 x and 1, whose rounding then pushes the same way row after row),
+// both terms are small.  A node x < 0 takes P_l(x) = (-1)^l P_l(-x): its odd rows
+// count with the other sign.  Error of (2l + 1) P_l against its value, RMS over all
+// rows and nodes at n = nl = 200, 1000, 6147: 1.7e-15, 8.0e-15, 4.1e-14; the
+// three-term form with a division in every step 7.8e-15, 3.3e-13, 3.7e-12, with
+// rounded coefficients for each row 6.3e-14, 3.6e-13, 4.1e-12.
+//
+// Lane i works out the row l0 + i (its division would otherwise be done by every
+// lane in every step) into LDS, from where all lanes read it.  From (D, P) = (1, 0)
+// the row of l = 0 (s = 0) yields P_0 = 1.
+__device__ __forceinline__ double legendre_row(int l) { return l == 0 ? 0.0 : 1.0 / l; }
+__device__ __forceinline__ double legendre_step(double s, double xm, double xm2, double &d,
+                                                double &p) {
+  d = fma(fma(-s, xm, xm2), p, fma(-s, d, d));
+  p += d;
   return p;
 }
 
 // One wave, 64 nodes.  Bound: the serial recurrence (one wave on each of n / 64
-// CUs, four FP64 operations a step): 123 us at nl = n = 6147, where the division in
-// every step and a load of cl_l waited for in it took 823 us.
+// CUs): 89 us at nl = n = 6147 (97 us as the three-term form with two rounded
+// coefficients for each row; with the division in every step and a load of cl_l
+// waited for in it 823 us).
 __global__ __launch_bounds__(64) void cl2corr_kernel(int nl, const double *__restrict__ cl, int n,
                                                      const double *__restrict__ x,
                                                      double *__restrict__ corr) {
-  __shared__ double2 ab[2][64];
+  __shared__ double row[2][64];
   __shared__ double c[2][64];
   const int lane = threadIdx.x, k = blockIdx.x * 64 + lane;
   const double xk = x[min(k, n - 1)];
+  const double xm = fabs(xk) - 1.0, xm2 = 2.0 * xm;
   auto fill = [&](int buf, int l0) {
     const int l = l0 + lane;
-    ab[buf][lane] = l < nl ? legendre_row(l) : double2{0.0, 0.0};
+    // rows past nl have c = 0 and s = 2, which only turns the sign of D: their
+    // values stay finite where P_l grows without bound (|x| > 1)
+    row[buf][lane] = l < nl ? legendre_row(l) : 2.0;
     c[buf][lane] = l < nl ? cl[l] * (double(2 * l + 1) / (4.0 * M_PI)) : 0.0;
   };
-  double p0 = 1.0, p1 = 0.0, acc = 0.0;
+  double d = 1.0, p = 0.0, acc[2] = {0.0, 0.0};  // sums of the even and odd rows
   int buf = 0;
   fill(0, 0);
   __syncthreads();
   for (int l0 = 0; l0 < nl; l0 += 64, buf ^= 1) {
     if (l0 + 64 < nl) fill(buf ^ 1, l0 + 64);
     // 16 rows to registers while the 16 before them are run: a wave that is
-    // alone on its CU hides no latency; rows past nl have c = 0 and values of
-    // zero (a node with |x| > 1, where P_l grows without bound, must not
-    // overflow in them)
-    double2 r[4][16];
+    // alone on its CU hides no latency
+    double r[4][16];
     double cv[4][16];
 #pragma unroll
     for (int q = 0; q <= 4; ++q) {
       if (q < 4) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          r[q][j] = ab[buf][16 * q + j];
+          r[q][j] = row[buf][16 * q + j];
           cv[q][j] = c[buf][16 * q + j];
         }
       }
@@ -112,49 +119,51 @@ __global__ __launch_bounds__(64) void cl2corr_kernel(int nl, const double *__res
       if (q > 0) {
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-          acc = fma(cv[q - 1][j], legendre_step(r[q - 1][j], xk, p0, p1), acc);
+          acc[j & 1] = fma(cv[q - 1][j], legendre_step(r[q - 1][j], xm, xm2, d, p), acc[j & 1]);
       }
     }
     __syncthreads();
   }
-  if (k < n) corr[k] = acc;
+  if (k < n) corr[k] = xk < 0.0 ? acc[0] - acc[1] : acc[0] + acc[1];
 }
 
 // part[wave][l]: 2 pi sum over the wave's nodes of w_k corr_k P_l(x_k), 32 rows
 // of l reduced over the wave at a time.  Bound as above, the reduction adding
-// half: 165 us at n = nl = 6147 (a shuffle butterfly for every l: 2076 us).
+// half: 159 us at n = nl = 6147 (a shuffle butterfly for every l: 2076 us).
 __global__ __launch_bounds__(64) void corr2cl_kernel(int n, const double *__restrict__ x,
                                                      const double *__restrict__ w,
                                                      const double *__restrict__ corr, int nl,
                                                      double *__restrict__ part) {
-  __shared__ double2 ab[2][32];
+  __shared__ double row[2][32];
   const int lane = threadIdx.x, k = blockIdx.x * 64 + lane;
   const bool ok = k < n;
-  const double xk = ok ? x[k] : 0.0;
+  const double xk = ok ? x[k] : 1.0;
+  const double xm = fabs(xk) - 1.0, xm2 = 2.0 * xm;
   const double a = ok ? 2.0 * M_PI * w[k] * corr[k] : 0.0;
+  const double ap[2] = {a, xk < 0.0 ? -a : a};  // for even and odd rows
   double *__restrict__ out = part + int64_t(blockIdx.x) * nl;
   auto fill = [&](int buf, int l0) {
-    if (lane < 32) ab[buf][lane] = legendre_row(l0 + lane);
+    if (lane < 32) row[buf][lane] = legendre_row(l0 + lane);
   };
-  double p0 = 1.0, p1 = 0.0;
+  double d = 1.0, p = 0.0;
   int buf = 0;
-  double2 r[32];  // rows 0..15 of a turn are loaded before the reduction of the last one
+  double r[32];  // rows 0..15 of a turn are loaded before the reduction of the last one
   fill(0, 0);
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < 16; ++j) r[j] = ab[0][j];
+  for (int j = 0; j < 16; ++j) r[j] = row[0][j];
   for (int l0 = 0; l0 < nl; l0 += 32) {
 #pragma unroll
-    for (int j = 16; j < 32; ++j) r[j] = ab[buf][j];
+    for (int j = 16; j < 32; ++j) r[j] = row[buf][j];
     buf ^= 1;
     fill(buf, l0 + 32);
     __builtin_amdgcn_sched_barrier(0);
     double v[32];
 #pragma unroll
-    for (int j = 0; j < 32; ++j) v[j] = a * legendre_step(r[j], xk, p0, p1);
+    for (int j = 0; j < 32; ++j) v[j] = ap[j & 1] * legendre_step(r[j], xm, xm2, d, p);
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 16; ++j) r[j] = ab[buf][j];
+    for (int j = 0; j < 16; ++j) r[j] = row[buf][j];
     __builtin_amdgcn_sched_barrier(0);
     const double s = wave_sums32(v, lane);
     const int l = l0 + (lane >> 1);
