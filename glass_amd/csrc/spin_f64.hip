@@ -6,18 +6,17 @@
 // ring of a pair follows from F+(pi - t) = sigma F+(t), F-(pi - t) = -sigma F-(t),
 // sigma = (-1)^(l+m+s).
 //
-// A lane owns one ring pair of one m and runs both recurrences.  The sums are
-// linear in lambda, so it accumulates lambda+ and lambda- against E and B as
-// they come (eight FMAs a step, split by the parity of l - m, which is static
-// in the unrolled loop) and forms Q and U once, after the loop; the two
+// A lane owns one ring pair of one m and runs both recurrences from l0 = max(m, s).
+// The sums are linear in lambda, so it accumulates lambda+ and lambda- against E
+// and B as they come (eight FMAs a step, split by the parity of l - l0, which is
+// static in the unrolled loop) and forms Q and U once, after the loop; the two
 // recurrence steps cost six more operations.  E, B and the recurrence
 // coefficients are wave-uniform and arrive by scalar loads, kChunk rows at a
-// time.  Values far below the range that matters are kept scaled
+// time.  Coefficients below the spin (l < s, which a spin-s field does not have)
+// are not read.  Values far below the range that matters are kept scaled
 // (to_scaled_low) and rescaled once per chunk, so no step has a test.  Skipping
 // the sums while a whole wave is scaled would save 1 to 5 % (nside 300, 1024),
-// but a coefficient that is not finite would then not reach every ring.  The
-// coefficients below the spin (l < s, which a spin-s field does not have) never
-// enter a sum, whatever they hold.
+// but a coefficient that is not finite would then not reach every ring.
 //
 // Bound: FP64 issue, 14 operations per (l, m, ring pair).  Measured at nside
 // 300, lmax 767 (E and B): 141 us (chunks of 4 rows 169 us, two ring pairs per
@@ -36,7 +35,7 @@ constexpr int kChunk = 8;  // rows per batch of scalar loads
 struct spin_state {
   double x, a0, a1, b0, b1;  // (l-2, l-1) of +s and -s
   int kp, km;
-  // [parity of l - m]: lambda+ E, lambda+ B, lambda- E, lambda- B
+  // [parity of l - l0]: lambda+ E, lambda+ B, lambda- E, lambda- B
   double2 pe[2], pb[2], me[2], mb[2];
 
   // one recurrence step; the new values are in a1, b1
@@ -98,14 +97,11 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
     to_scaled_low(v, (long long)kp.y + es1 + ec1 + t, sp, s.kp);
     v = frexp(km.x * ms2 * mc2, &t);
     to_scaled_low(v, (long long)km.y + es2 + ec2 + t, sm, s.km);
-    // the (0, 0, -1) row at l0 turns (seed, 0) into the seed; for l0 = m + 1 the
-    // loop starts at m, one such row earlier, to keep its parity
-    const bool odd = (l0 - m) & 1;
+    // the (0, 0, -1) row at l0 turns (seed, 0) into the seed
     s.x = x;
-    s.a0 = odd ? 0.0 : sp;
-    s.a1 = odd ? sp : 0.0;
-    s.b0 = odd ? 0.0 : sm;
-    s.b1 = odd ? sm : 0.0;
+    s.a0 = sp;
+    s.b0 = sm;
+    s.a1 = s.b1 = 0.0;
 #pragma unroll
     for (int p = 0; p < 2; ++p)
       s.pe[p] = s.pb[p] = s.me[p] = s.mb[p] = double2{0.0, 0.0};
@@ -115,8 +111,7 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
   const double *__restrict__ cf = tab + 3 * base;
   const double2 *__restrict__ e = E + base, *__restrict__ b = B + base;
   const int nl = lmax + 1 - m;
-  const int first = l0 - m;  // the first row of the sums
-  int i = first & ~1;
+  int i = l0 - m;
   bool scaled = s.any_scaled();  // wave-uniform
   for (; i + kChunk <= nl; i += kChunk) {
     double c[3 * kChunk];
@@ -127,7 +122,6 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
     for (int q = 0; q < kChunk; ++q) ev[q] = e[i + q];
 #pragma unroll
     for (int q = 0; q < kChunk; ++q) bv[q] = b[i + q];
-    if (i < first) ev[0] = bv[0] = double2{0.0, 0.0};  // l = l0 - 1, below the spin
 #pragma unroll
     for (int q = 0; q < kChunk; ++q) {
       s.advance(c[3 * q], c[3 * q + 1], c[3 * q + 2]);
@@ -139,11 +133,10 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
     }
   }
 #pragma unroll
-  for (int q = 0; q < kChunk - 1; ++q)  // the last rows (the chunks leave i even)
+  for (int q = 0; q < kChunk - 1; ++q)  // the last rows
     if (i + q < nl) {
       s.advance(cf[3 * (i + q)], cf[3 * (i + q) + 1], cf[3 * (i + q) + 2]);
-      const bool below = q == 0 && i < first;
-      s.add(q & 1, below ? double2{0.0, 0.0} : e[i + q], below ? double2{0.0, 0.0} : b[i + q]);
+      s.add(q & 1, e[i + q], b[i + q]);
     }
 
   const double sg = (spin & 1) ? -1.0 : 1.0;
@@ -154,7 +147,7 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
   double ps = 0.0, pc = 1.0;
   if (pnum) sincospi(2.0 * double((int64_t(m) * pnum) % pden) / double(pden), &ps, &pc);
   const cplx<double> ph = {pc, ps};
-  cplx<double> qa[2], qb[2], ua[2], ub[2];  // by the parity of l - m
+  cplx<double> qa[2], qb[2], ua[2], ub[2];  // by the parity of l - l0
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     double2 PE = s.pe[p], PB = s.pb[p], ME = s.me[p], MB = s.mb[p];
@@ -168,7 +161,8 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
     ua[p] = pB;
     ub[p] = cplx<double>{mE.im, -mE.re};  // -i E F-
   }
-  // sigma = (-1)^(l + m + s) = sg on even, -sg on odd l - m
+  // sigma = (-1)^(l + m + s) = south on even, -south on odd l - l0
+  const double south = ((l0 + m + spin) & 1) ? -1.0 : 1.0;
   const cplx<double> qn = cadd(cadd(qa[0], qb[0]), cadd(qa[1], qb[1]));
   const cplx<double> un = cadd(cadd(ua[0], ub[0]), cadd(ua[1], ub[1]));
   const cplx<double> qs = cadd(csub(qa[0], qb[0]), csub(qb[1], qa[1]));
@@ -180,8 +174,8 @@ __global__ __launch_bounds__(256) void spin_synth_f64_kernel(
   if (rp < npairs - 1) {
     const cplx<double> q1 = cmul(qs, ph), u1 = cmul(us, ph);
     o = Fo + int64_t(nrings - 1 - rp) * stride + 2 * m;
-    o[0] = double2{sg * q1.re, sg * q1.im};
-    o[1] = double2{sg * u1.re, sg * u1.im};
+    o[0] = double2{south * q1.re, south * q1.im};
+    o[1] = double2{south * u1.re, south * u1.im};
   }
 }
 
