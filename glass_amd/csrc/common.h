@@ -148,7 +148,6 @@ struct ga_plan {
   // lambda_l = a (x lambda_{l-1} - b lambda_{l-2}); seed constants c_m with
   // lambda_mm = c_m sin^m theta
   double2 *d_ab = nullptr;
-  double2 *d_aab = nullptr;  // (a, a b) per (l, m): the same recurrence, one FMA deep
   // The split-FP16 synthesis runs the recurrence on y_l = lambda_l / c_l with
   // c_m = c_{m+1} = 1, c_l = a_l b_l c_{l-2}, which makes the lambda_{l-2}
   // coefficient 1: y_l = (gam_l x) y_{l-1} - y_{l-2}, gam_l = a_l c_{l-1} / c_l
@@ -158,6 +157,11 @@ struct ga_plan {
   // max_l sqrt((2l+1)/4pi) / c_l times it below 2^15.5 (FP16 range).
   double *d_gam = nullptr;
   double *d_csc = nullptr;
+  // The same form for the FP64 stages, worked out in extended precision:
+  // d_h64 = gam_l / 2 - 1, so that gam_l x = fma(h, 2x, 2x) is rounded once and its
+  // table is exact to far below that, and d_c64 = c_l (d_h64 padded by 64)
+  double *d_h64 = nullptr;
+  double *d_c64 = nullptr;
   int lam_exp16 = 8;
   double *d_cm = nullptr;
   // FP16 MFMA stage: l-slabs of kSlab rows per m; slab_off[m] = index of the

@@ -159,6 +159,39 @@ __device__ __forceinline__ void rescale_low(double &p0, double &p1, int &k) {
   k += up;
 }
 
+// One row of the normalised recurrence of the FP64 stages, X = 2x, h = gam / 2 - 1
+// (d_h64); the new value is in p1.  Two operations: the coefficient gam x, rounded
+// once, and the step, from (p0, p1) = (y_{l-2}, y_{l-1}).  The row of l = m (h = -1)
+// yields the seed from p1 = 0 and p0 = -seed.
+//
+// For m = 0, 1 the coefficients tend to 2x so fast that the rounding of gam x is the
+// same for most rows, which adds up over a long recurrence.  There DIFF carries
+// the difference p0 = y_{l-1} - y_{l-2} (at first the seed), with gam x - 2 as its
+// coefficient, for one operation more (map2alm without iterations at nside 512,
+// lmax 1023: 171 -> 178 us, the workgroup of m = 0 being the longest).  Below lmax
+// 832 the whole error stays under that of the (a, b) form without it (nside 512,
+// lmax 820: 0.9556e-14 against 0.9553e-14; lmax 880: 1.027e-14 against 1.017e-14).
+//
+// Error of lambda, RMS over all (l, m) and rings (weighted by their pixels), at
+// nside 64, lmax 128; 256, 512; 512, 1023; 1024, 2048: as a (x lambda_{l-1} - b
+// lambda_{l-2}) 2.06e-15, 6.2e-15, 1.17e-14, 2.28e-14; this form 1.91e-15, 6.0e-15,
+// 1.15e-14, 2.25e-14 (without DIFF 1.21e-14 and 2.38e-14 in the last two); with
+// gam and c from products in double precision 2.81e-15, 7.9e-15, 1.41e-14, 3.04e-14.
+// Most of what is left is the seed's (sin^m by repeated squaring).
+__device__ __forceinline__ bool norm_diff(int lmax, int m) { return m < 2 && lmax >= 832; }
+
+template <bool DIFF>
+__device__ __forceinline__ void norm_step(double h, double X, double &p0, double &p1) {
+  if (DIFF) {
+    p0 = fma(fma(1.0 + h, X, -2.0), p1, p0);
+    p1 += p0;
+  } else {
+    const double y = fma(fma(h, X, X), p1, -p0);
+    p0 = p1;
+    p1 = y;
+  }
+}
+
 // ---- sums over the lanes of a wave
 template <int CTRL>
 __device__ __forceinline__ double dpp_move(double v) {

@@ -21,6 +21,7 @@
 // 878 us (a butterfly of each sum through LDS shuffles: 4803 us); nside 256,
 // lmax 512: 48 us (482 us).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "device.h"
@@ -34,11 +35,30 @@ constexpr int kRows = 16;        // l rows per reduction
 constexpr int kSums = 2 * kRows;  // (re, im) of each
 static_assert(kSums == 32, "wave_sums32");
 
+// the values of kRows rows on the wave's ring pairs and each lane's part of their
+// sums (re, im)
+template <int RPL, bool DIFF>
+__device__ __forceinline__ void anal_rows(const double (&h)[kRows], const double (&X)[RPL],
+                                          double (&p0)[RPL], double (&p1)[RPL],
+                                          const double2 (&q)[2][RPL], double (&v)[kSums]) {
+#pragma unroll
+  for (int i = 0; i < kRows; ++i) {
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      norm_step<DIFF>(h[i], X[j], p0[j], p1[j]);
+      const double y = p1[j];
+      v[2 * i] = j == 0 ? y * q[i & 1][j].x : fma(y, q[i & 1][j].x, v[2 * i]);
+      v[2 * i + 1] = j == 0 ? y * q[i & 1][j].y : fma(y, q[i & 1][j].y, v[2 * i + 1]);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // rows in order: registers
+  }
+}
+
 template <int RPL>
 __global__ __launch_bounds__(256, RPL == 8 ? 2 : 3) void legendre_anal_f64_kernel(
     int lmax, int npairs, int nrings, int nrg, const double *__restrict__ z,
-    const double *__restrict__ sth, const double *__restrict__ gam,
-    const double *__restrict__ csc, const double *__restrict__ cm,
+    const double *__restrict__ sth, const double *__restrict__ h,
+    const double *__restrict__ c, const double *__restrict__ cm,
     const double2 *__restrict__ F, double *__restrict__ out /* [slot][idx] (re, im) */,
     int64_t slot_stride, int accumulate) {
   __shared__ double red[2][4][kSums];
@@ -48,17 +68,18 @@ __global__ __launch_bounds__(256, RPL == 8 ? 2 : 3) void legendre_anal_f64_kerne
   const int rp0 = (rg * nw + wave) * 64 * RPL + lane;
   const int64_t base = hp_index(lmax, m, m);
 
-  double x[RPL], p0[RPL], p1[RPL];
+  const bool diff = norm_diff(lmax, m);
+  double X[RPL], p0[RPL], p1[RPL];
   int k[RPL];
   double2 q[2][RPL];
 #pragma unroll
   for (int j = 0; j < RPL; ++j) {
     const int rp = rp0 + 64 * j;
     const int rpc = min(rp, npairs - 1);
-    x[j] = z[rpc];
+    X[j] = 2.0 * z[rpc];
     p1[j] = 0.0;
     legendre_seed_low(cm[m], sth[rpc], m, p0[j], k[j]);
-    p0[j] = -p0[j];  // (-seed, 0): the first step (gam = 0) yields the seed
+    if (!diff) p0[j] = -p0[j];  // the first row (h = -1) yields the seed
     double2 fn = {0.0, 0.0}, fs = {0.0, 0.0};
     if (rp < npairs) fn = F[int64_t(rp) * (lmax + 1) + m];
     if (rp < npairs - 1) fs = F[int64_t(nrings - 1 - rp) * (lmax + 1) + m];
@@ -66,55 +87,47 @@ __global__ __launch_bounds__(256, RPL == 8 ? 2 : 3) void legendre_anal_f64_kerne
     q[1][j] = double2{fn.x - fs.x, fn.y - fs.y};
   }
 
-  const double *__restrict__ g = gam + base;
+  h += base;
   const int nl = lmax + 1 - m;
   bool scaled = true;  // wave-uniform: some value of the wave may still be scaled
   out += 2 * (int64_t(rg) * slot_stride + base);
-  int buf = 0, turn = 0;
   // the coefficient table is padded: the rows past lmax in the last turn are
   // computed and not stored
-  for (int i0 = 0; i0 < nl; i0 += kRows) {
-    double gv[kRows];
+  auto all_rows = [&](auto form) {
+    int buf = 0, turn = 0;
+    for (int i0 = 0; i0 < nl; i0 += kRows) {
+      double hv[kRows], v[kSums];
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) gv[i] = g[i0 + i];
-    double v[kSums];
+      for (int i = 0; i < kRows; ++i) hv[i] = h[i0 + i];
+      anal_rows<RPL, form.value>(hv, X, p0, p1, q, v);
+      const double sum = wave_sums32(v, lane);
+      if (!(lane & 1)) red[buf][wave][lane >> 1] = sum;
+      if (scaled) {
+        bool any = false;
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-#pragma unroll
-      for (int j = 0; j < RPL; ++j) {
-        const double y = fma(gv[i] * x[j], p1[j], -p0[j]);
-        p0[j] = p1[j];
-        p1[j] = y;
-        v[2 * i] = j == 0 ? y * q[i & 1][j].x : fma(y, q[i & 1][j].x, v[2 * i]);
-        v[2 * i + 1] = j == 0 ? y * q[i & 1][j].y : fma(y, q[i & 1][j].y, v[2 * i + 1]);
+        for (int j = 0; j < RPL; ++j) {
+          rescale_low(p0[j], p1[j], k[j]);
+          any |= k[j] < 0;
+        }
+        scaled = wave_any(any);
       }
-      __builtin_amdgcn_sched_barrier(0);  // rows in order: registers
-    }
-    const double sum = wave_sums32(v, lane);
-    if (!(lane & 1)) red[buf][wave][lane >> 1] = sum;
-    if (scaled) {
-      bool any = false;
-#pragma unroll
-      for (int j = 0; j < RPL; ++j) {
-        rescale_low(p0[j], p1[j], k[j]);
-        any |= k[j] < 0;
+      __syncthreads();
+      if (wave == turn && lane < kSums) {
+        double s = red[buf][0][lane];
+        for (int w = 1; w < nw; ++w) s += red[buf][w][lane];
+        const int i = i0 + (lane >> 1);
+        if (i < nl) {
+          s = (m == 0 && (lane & 1)) ? 0.0 : s * c[base + i];
+          double *o = out + 2 * int64_t(i0) + lane;
+          *o = accumulate ? *o + s : s;
+        }
       }
-      scaled = wave_any(any);
+      buf ^= 1;  // the other buffer was read before this turn's barrier
+      turn = turn + 1 == nw ? 0 : turn + 1;
     }
-    __syncthreads();
-    if (wave == turn && lane < kSums) {
-      double s = red[buf][0][lane];
-      for (int w = 1; w < nw; ++w) s += red[buf][w][lane];
-      const int i = i0 + (lane >> 1);
-      if (i < nl) {
-        s = (m == 0 && (lane & 1)) ? 0.0 : s * csc[base + i];
-        double *o = out + 2 * int64_t(i0) + lane;
-        *o = accumulate ? *o + s : s;
-      }
-    }
-    buf ^= 1;  // the other buffer was read before this turn's barrier
-    turn = turn + 1 == nw ? 0 : turn + 1;
-  }
+  };
+  if (diff) all_rows(std::true_type());
+  else all_rows(std::false_type());
 }
 
 }  // namespace
@@ -136,7 +149,7 @@ int launch_legendre_anal_f64(const ga_plan *p, const double *F, double *alm, dou
 #define GA_ANAL64(RPL_)                                                                          \
   hipLaunchKernelGGL(legendre_anal_f64_kernel<RPL_>, dim3(m_run8_blocks(p->lmax, nrg)),           \
                      dim3(64 * nw), 0, stream, p->lmax, p->npairs, p->nrings, nrg, p->d_z,        \
-                     p->d_sth, p->d_gam, p->d_csc, p->d_cm, reinterpret_cast<const double2 *>(F), \
+                     p->d_sth, p->d_h64, p->d_c64, p->d_cm, reinterpret_cast<const double2 *>(F), \
                      out, p->nalm, nrg == 1 && accumulate)
   if (rpl == 1) GA_ANAL64(1);
   else if (rpl == 2) GA_ANAL64(2);

@@ -355,19 +355,22 @@ extern "C" int ga_plan_create(int32_t nside, int32_t lmax, ga_plan **out) {
       // and only feed recurrence steps after that m's last row, whose values
       // are discarded
       std::vector<double> gam(size_t(p->nalm + 64), 0.0), csc(size_t(p->nalm + 4), 1.0);
+      std::vector<double> amp(size_t(lmax + 1));  // sqrt((2l + 1) / (4 pi))
+      for (int64_t l = 0; l <= lmax; ++l)
+        amp[size_t(l)] = std::sqrt((2.0 * double(l) + 1.0) / (4.0 * M_PI));
       double bound = 0.0;
       for (int64_t m = 0; m <= lmax; ++m) {
         const int64_t b0 = hp_index(lmax, m, m);
         double cprev2 = 1.0, cprev = 1.0;  // c_{l-2}, c_{l-1}
         gam[size_t(b0)] = 0.0;
         csc[size_t(b0)] = 1.0;
-        bound = std::max(bound, std::sqrt((2.0 * double(m) + 1.0) / (4.0 * M_PI)));
+        bound = std::max(bound, amp[size_t(m)]);
         for (int64_t l = m + 1; l <= lmax; ++l) {
           const double2 v = ab[size_t(b0 + (l - m))];
           const double c = l == m + 1 ? 1.0 : v.x * v.y * cprev2;
           gam[size_t(b0 + (l - m))] = v.x * cprev / c;
           csc[size_t(b0 + (l - m))] = c;
-          bound = std::max(bound, std::sqrt((2.0 * double(l) + 1.0) / (4.0 * M_PI)) / c);
+          bound = std::max(bound, amp[size_t(l)] / c);
           cprev2 = cprev;
           cprev = c;
         }
@@ -377,11 +380,29 @@ extern "C" int ga_plan_create(int32_t nside, int32_t lmax, ga_plan **out) {
       p->lam_exp16 = e;
       if ((rc = upload(&p->d_gam, gam.data(), gam.size() * 8, &p->table_bytes))) return fail(rc);
       if ((rc = upload(&p->d_csc, csc.data(), csc.size() * 8, &p->table_bytes))) return fail(rc);
+      // The same for the FP64 stages, in extended precision and over the same
+      // arrays: with A_l = a_l^2 = (4 l^2 - 1) / (l^2 - m^2) and b_l = 1 / a_{l-1},
+      //   gam_{m+1} = a_{m+1}, gam_l = A_{l-1} / gam_{l-1},  c_l^2 = c_{l-2}^2 A_l / A_{l-1}
+      // (the integer products are exact)
+      for (int64_t m = 0; m <= lmax; ++m) {
+        double *h = gam.data() + hp_index(lmax, m, m), *c = csc.data() + hp_index(lmax, m, m);
+        long double g = std::sqrt((long double)(2 * m + 3)), k0 = 1.0L, k1 = 1.0L;  // c^2 of l-2, l-1
+        h[0] = -1.0;
+        if (m < lmax) h[1] = double(0.5L * g - 1.0L);
+        for (int64_t l = m + 2; l <= lmax; ++l) {
+          const int64_t n1 = 4 * (l - 1) * (l - 1) - 1, d1 = (l - 1) * (l - 1) - m * m;
+          const int64_t n = 4 * l * l - 1, d = l * l - m * m;
+          g = (long double)n1 / ((long double)d1 * g);
+          const long double k = k0 * ((long double)(n * d1) / (long double)(d * n1));
+          h[l - m] = double(0.5L * g - 1.0L);
+          c[l - m] = std::sqrt(double(k));
+          k0 = k1;
+          k1 = k;
+        }
+      }
+      if ((rc = upload(&p->d_h64, gam.data(), gam.size() * 8, &p->table_bytes))) return fail(rc);
+      if ((rc = upload(&p->d_c64, csc.data(), csc.size() * 8, &p->table_bytes))) return fail(rc);
     }
-    // the same recurrence as (a, a b): lambda_l = (a x) lambda_{l-1} - (a b) lambda_{l-2},
-    // one FMA on the dependency chain per step
-    for (double2 &v : ab) v.y *= v.x;
-    if ((rc = upload(&p->d_aab, ab.data(), ab.size() * sizeof(double2), &p->table_bytes))) return fail(rc);
     // c_m = (-1)^m sqrt((2m+1)/(4 pi) prod_{k<=m} (2k-1)/(2k)): lambda_mm = c_m sin^m
     std::vector<double> cm(size_t(lmax + 1));
     long double acc = 1.0L;
@@ -544,7 +565,8 @@ extern "C" int ga_plan_create(int32_t nside, int32_t lmax, ga_plan **out) {
 extern "C" int ga_plan_destroy(ga_plan *p) {
   if (!p) return GA_OK;
   void *ptrs[] = {p->d_z, p->d_sth, p->d_ring_start, p->d_ring_n, p->d_ring_pnum, p->d_ring_pden,
-                  p->d_ab, p->d_aab, p->d_gam, p->d_csc, p->d_cm, p->d_slab_off, p->d_spin[0], p->d_spin[1], p->d_spin[2],
+                  p->d_ab, p->d_gam, p->d_csc, p->d_h64, p->d_c64, p->d_cm, p->d_slab_off, p->d_spin[0],
+                  p->d_spin[1], p->d_spin[2],
                   p->d_spin_seed[0], p->d_spin_seed[1], p->d_spin_seed[2], p->d_blu_off,
                   p->d_blu64, p->d_blu32, p->d_tw64, p->d_tw32, p->d_rings_pow2,
                   p->d_rings_blu, p->d_rings_wide, p->d_rings_narrow, p->d_rings_bwide,
