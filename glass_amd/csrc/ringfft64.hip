@@ -438,9 +438,10 @@ int launch_ring_synth_f64(const ga_plan *p, int S, const double *F, double *maps
 
 int launch_ring_anal_f64(const ga_plan *p, const double *maps, const double *pixw, double wc,
                          double *F, hipStream_t s) {
-  // the analysis holds a whole ring in registers and LDS: nside up to 2048
-  GA_REQUIRE(size_t(padded_len<float>(std::max(p->max_L, 4 * p->nside))) * sizeof(c64) <= 160 * 1024,
-             GA_ERR_UNSUPPORTED, "ring analysis: nside %d too large", p->nside);
+  // the largest nside whose belt ring, padded, fits LDS as a whole, which is the
+  // limit of the entry point; the kernel holds at most half a ring there (136 KB at
+  // nside 4096, checked in launch_anal64)
+  GA_REQUIRE(p->nside <= 2482, GA_ERR_UNSUPPORTED, "ring analysis: nside %d too large", p->nside);
   GA_RING64_SIZES(launch_anal64, p, maps, pixw, wc, F, s);
 }
 
