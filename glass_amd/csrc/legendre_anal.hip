@@ -36,13 +36,14 @@ __device__ __forceinline__ float wave_sum_last(float v) {
   v = dpp_add<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
   return v;                    // lane 63: the wave's sum
 }
+
 constexpr int kAnalRPL = 8;  // ring pairs per lane
 
-template <typename T, int SC>
+template <int SC>
 __global__ __launch_bounds__(256) void legendre_anal_kernel(
     int lmax, int npairs, int nrings, int S, const double *__restrict__ z,
     const double *__restrict__ sth, const double2 *__restrict__ ab, const double *__restrict__ cm,
-    const cplx<T> *__restrict__ F, cplx<T> *__restrict__ partial, int64_t nalm) {
+    const cplx<float> *__restrict__ F, cplx<float> *__restrict__ partial, int64_t nalm) {
   constexpr int RPL = kAnalRPL;
   const int m = blockIdx.x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(256) void legendre_anal_kernel(
 
   double x[RPL], p0[RPL], p1[RPL];
   int kk[RPL];
-  cplx<T> qe[RPL][SC], qo[RPL][SC];
+  cplx<float> qe[RPL][SC], qo[RPL][SC];
 #pragma unroll
   for (int j = 0; j < RPL; ++j) {
     const int rp = gw * 64 * RPL + j * 64 + lane;
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(256) void legendre_anal_kernel(
     legendre_seed(cm[m], sth[rpc], m, p0[j], kk[j]);
 #pragma unroll
     for (int c = 0; c < SC; ++c) {
-      cplx<T> fn = {T(0), T(0)}, fs = {T(0), T(0)};
+      cplx<float> fn = {0.0f, 0.0f}, fs = {0.0f, 0.0f};
       if (ok && s0 + c < S) {
         fn = F[(int64_t(rp) * (lmax + 1) + m) * S + s0 + c];
         if (rp < npairs - 1) fs = F[(int64_t(nrings - 1 - rp) * (lmax + 1) + m) * S + s0 + c];
@@ -74,13 +75,13 @@ __global__ __launch_bounds__(256) void legendre_anal_kernel(
       qo[j][c] = csub(fn, fs);
     }
   }
-  cplx<T> *out = partial + (int64_t(gw) * nalm + base) * S + s0;
+  cplx<float> *out = partial + (int64_t(gw) * nalm + base) * S + s0;
   for (int l = m; l <= lmax; ++l) {
     const double2 c = co[l - m];  // (1, -1) at l = m turns (seed, 0) into lambda_mm
     const bool odd = (l - m) & 1;
-    T acc_re[SC], acc_im[SC];
+    float acc_re[SC], acc_im[SC];
 #pragma unroll
-    for (int cc = 0; cc < SC; ++cc) { acc_re[cc] = T(0); acc_im[cc] = T(0); }
+    for (int cc = 0; cc < SC; ++cc) { acc_re[cc] = 0.0f; acc_im[cc] = 0.0f; }
     bool any_on = false;
 #pragma unroll
     for (int j = 0; j < RPL; ++j) {
@@ -88,11 +89,11 @@ __global__ __launch_bounds__(256) void legendre_anal_kernel(
       p0[j] = p1[j];
       p1[j] = pn;
       if (kk[j] < 0 && fabs(p1[j]) > 0x1p300) { p1[j] *= 0x1p-600; p0[j] *= 0x1p-600; ++kk[j]; }
-      const T v = kk[j] == 0 ? T(p1[j]) : T(0);
+      const float v = kk[j] == 0 ? float(p1[j]) : 0.0f;
       any_on |= kk[j] == 0;
 #pragma unroll
       for (int cc = 0; cc < SC; ++cc) {
-        const cplx<T> q = odd ? qo[j][cc] : qe[j][cc];
+        const cplx<float> q = odd ? qo[j][cc] : qe[j][cc];
         acc_re[cc] += v * q.re;
         acc_im[cc] += v * q.im;
       }
@@ -107,7 +108,8 @@ __global__ __launch_bounds__(256) void legendre_anal_kernel(
     if (lane == 63) {
 #pragma unroll
       for (int cc = 0; cc < SC; ++cc)
-        if (s0 + cc < S) out[int64_t(l - m) * S + cc] = cplx<T>{acc_re[cc], m == 0 ? T(0) : acc_im[cc]};
+        if (s0 + cc < S)
+          out[int64_t(l - m) * S + cc] = cplx<float>{acc_re[cc], m == 0 ? 0.0f : acc_im[cc]};
     }
   }
 }
@@ -129,14 +131,15 @@ __global__ void reduce_partials_kernel(int64_t n, int nw, const cplx<T> *__restr
 // F+- = -(sY +- (-1)^s (-s)Y) / 2; south ring via F+(pi - t) = sigma F+(t),
 // F-(pi - t) = -sigma F-(t), sigma = (-1)^(l+m+s).
 
-template <typename T, int SC>
+template <int SC>
 __global__ __launch_bounds__(256) void spin_synth_kernel(
     int lmax, int npairs, int nrings, int spin, int S, const double *__restrict__ z,
     const double *__restrict__ sth, const double *__restrict__ tab /* (A,B,C) per (l,m) */,
     const double2 *__restrict__ seedk /* per m: (+s mant, +s exp), */,
     const double2 *__restrict__ seedkm /* per m: (-s mant, -s exp) */,
     const int32_t *__restrict__ ring_pnum, const int32_t *__restrict__ ring_pden,
-    const cplx<T> *__restrict__ E, const cplx<T> *__restrict__ B, cplx<T> *__restrict__ Fo) {
+    const cplx<float> *__restrict__ E, const cplx<float> *__restrict__ B,
+    cplx<float> *__restrict__ Fo) {
   const int m = blockIdx.x;
   const int rp = blockIdx.y * blockDim.x + threadIdx.x;
   const int s0 = blockIdx.z * SC;
@@ -144,11 +147,11 @@ __global__ __launch_bounds__(256) void spin_synth_kernel(
   const double x = z[rpc], st = sth[rpc];
   const int l0 = m > spin ? m : spin;
   // accumulators [shell][QA, QB, UA, UB] x [parity class of l + m + s]
-  cplx<T> acc[SC][4][2];
+  cplx<float> acc[SC][4][2];
 #pragma unroll
   for (int c = 0; c < SC; ++c)
 #pragma unroll
-    for (int a = 0; a < 4; ++a) acc[c][a][0] = acc[c][a][1] = cplx<T>{T(0), T(0)};
+    for (int a = 0; a < 4; ++a) acc[c][a][0] = acc[c][a][1] = cplx<float>{0.0f, 0.0f};
 
   if (l0 <= lmax) {
     double sh = sqrt(0.5 * (1.0 - x)), ch = sqrt(0.5 * (1.0 + x));
@@ -184,19 +187,19 @@ __global__ __launch_bounds__(256) void spin_synth_kernel(
       if (kp_ < 0 && fabs(a1) > 0x1p300) { a1 *= 0x1p-600; a0 *= 0x1p-600; ++kp_; }
       if (km_ < 0 && fabs(b1) > 0x1p300) { b1 *= 0x1p-600; b0 *= 0x1p-600; ++km_; }
       const double lp = kp_ == 0 ? a1 : 0.0, lm = km_ == 0 ? b1 : 0.0;
-      const T fp = T(-0.5 * (lp + sgn * lm)), fm = T(-0.5 * (lp - sgn * lm));
+      const float fp = float(-0.5 * (lp + sgn * lm)), fm = float(-0.5 * (lp - sgn * lm));
       const int par = (l + m + spin) & 1;
       const int64_t ia = (base + (l - m)) * S + s0;
 #pragma unroll
       for (int c = 0; c < SC; ++c) {
         if (s0 + c >= S) break;
-        cplx<T> e = E[ia + c], b = B[ia + c];
-        if (m == 0) { e.im = T(0); b.im = T(0); }
+        cplx<float> e = E[ia + c], b = B[ia + c];
+        if (m == 0) { e.im = 0.0f; b.im = 0.0f; }
         // QA += E F+, QB += i B F-, UA += B F+, UB += -i E F-
-        acc[c][0][par] = cadd(acc[c][0][par], cplx<T>{e.re * fp, e.im * fp});
-        acc[c][1][par] = cadd(acc[c][1][par], cplx<T>{-b.im * fm, b.re * fm});
-        acc[c][2][par] = cadd(acc[c][2][par], cplx<T>{b.re * fp, b.im * fp});
-        acc[c][3][par] = cadd(acc[c][3][par], cplx<T>{e.im * fm, -e.re * fm});
+        acc[c][0][par] = cadd(acc[c][0][par], cplx<float>{e.re * fp, e.im * fp});
+        acc[c][1][par] = cadd(acc[c][1][par], cplx<float>{-b.im * fm, b.re * fm});
+        acc[c][2][par] = cadd(acc[c][2][par], cplx<float>{b.re * fp, b.im * fp});
+        acc[c][3][par] = cadd(acc[c][3][par], cplx<float>{e.im * fm, -e.re * fm});
       }
     }
   }
@@ -205,15 +208,17 @@ __global__ __launch_bounds__(256) void spin_synth_kernel(
   const int pnum = ring_pnum[rp], pden = ring_pden[rp];
   double ps = 0.0, pc = 1.0;
   if (pnum) sincospi(2.0 * double((int64_t(m) * pnum) % pden) / double(pden), &ps, &pc);
-  const cplx<T> ph = {T(pc), T(ps)};
+  const cplx<float> ph = {float(pc), float(ps)};
   // output ring buffer [ring][m][2S]: column 2s holds Q_s, 2s + 1 holds U_s
   const int64_t rowN = (int64_t(rp) * (lmax + 1) + m) * (2 * S) + 2 * s0;
   const int64_t rowS = (int64_t(nrings - 1 - rp) * (lmax + 1) + m) * (2 * S) + 2 * s0;
 #pragma unroll
   for (int c = 0; c < SC; ++c) {
     if (s0 + c >= S) break;
-    const cplx<T> qa_e = acc[c][0][0], qb_e = acc[c][1][0], qa_o = acc[c][0][1], qb_o = acc[c][1][1];
-    const cplx<T> ua_e = acc[c][2][0], ub_e = acc[c][3][0], ua_o = acc[c][2][1], ub_o = acc[c][3][1];
+    const cplx<float> qa_e = acc[c][0][0], qb_e = acc[c][1][0];
+    const cplx<float> qa_o = acc[c][0][1], qb_o = acc[c][1][1];
+    const cplx<float> ua_e = acc[c][2][0], ub_e = acc[c][3][0];
+    const cplx<float> ua_o = acc[c][2][1], ub_o = acc[c][3][1];
     Fo[rowN + 2 * c] = cmul(cadd(cadd(qa_e, qb_e), cadd(qa_o, qb_o)), ph);
     Fo[rowN + 2 * c + 1] = cmul(cadd(cadd(ua_e, ub_e), cadd(ua_o, ub_o)), ph);
     if (rp < npairs - 1) {
@@ -251,7 +256,7 @@ int launch_legendre_anal_f32(const ga_plan *p, int S, const float *F, float *alm
     const int nblk_y = (nw + 3) / 4;
     constexpr int SC = 2;
     dim3 grid(unsigned(p->lmax + 1), unsigned(nblk_y), unsigned((S + SC - 1) / SC));
-    hipLaunchKernelGGL((legendre_anal_kernel<float, SC>), grid, dim3(256), 0, stream, p->lmax,
+    hipLaunchKernelGGL((legendre_anal_kernel<SC>), grid, dim3(256), 0, stream, p->lmax,
                        p->npairs, p->nrings, S, p->d_z, p->d_sth, p->d_ab, p->d_cm,
                        (const cplx<float> *)F, (cplx<float> *)partial, p->nalm);
     GA_LAUNCH_CHECK();
@@ -259,24 +264,19 @@ int launch_legendre_anal_f32(const ga_plan *p, int S, const float *F, float *alm
   return launch_reduce(p->nalm * S, nw, partial, alm, accumulate, stream);
 }
 
-template <typename T>
-static int launch_spin(const ga_plan *p, int spin, int S, const T *E, const T *B, T *Fo,
-                       hipStream_t stream) {
+int launch_spin_synth_f32(const ga_plan *p, int spin, int S, const float *E, const float *B,
+                          float *Fo, hipStream_t stream) {
   GA_REQUIRE(spin >= 1 && spin <= 2 && p->d_spin[spin] && p->d_spin_seed[spin], GA_ERR_INVALID,
              "spin %d tables not prepared (call ga_plan_prepare_spin)", spin);
-  constexpr int SC = sizeof(T) == 8 ? 1 : 4;
+  constexpr int SC = 4;
   dim3 grid(unsigned(p->lmax + 1), unsigned((p->npairs + 255) / 256), unsigned((S + SC - 1) / SC));
-  hipLaunchKernelGGL((spin_synth_kernel<T, SC>), grid, dim3(256), 0, stream, p->lmax, p->npairs,
+  hipLaunchKernelGGL(spin_synth_kernel<SC>, grid, dim3(256), 0, stream, p->lmax, p->npairs,
                      p->nrings, spin, S, p->d_z, p->d_sth, p->d_spin[spin],
                      p->d_spin_seed[spin], p->d_spin_seed[spin] + (p->lmax + 1), p->d_ring_pnum,
-                     p->d_ring_pden, (const cplx<T> *)E, (const cplx<T> *)B, (cplx<T> *)Fo);
+                     p->d_ring_pden, (const cplx<float> *)E, (const cplx<float> *)B,
+                     (cplx<float> *)Fo);
   GA_LAUNCH_CHECK();
   return GA_OK;
-}
-
-int launch_spin_synth_f32(const ga_plan *p, int spin, int S, const float *E, const float *B,
-                          float *Fo, hipStream_t s) {
-  return launch_spin<float>(p, spin, S, E, B, Fo, s);
 }
 
 }  // namespace ga

@@ -37,8 +37,8 @@ namespace {
 
 // In-place forward FFT (e^{-2 pi i}), natural order in, bit-reversed out, on P
 // arrays X + p ldx at once (one barrier per stage for all of them).
-template <typename T, int NT, int P>
-__device__ void fft_dif(cplx<T> *X, int ldx, int L, const typename tab_t<T>::type *tw, int maxL) {
+template <int NT, int P>
+__device__ void fft_dif(cplx<float> *X, int ldx, int L, const float2 *tw, int maxL) {
   const int t = threadIdx.x;
   const int logL = ilog2(L);
   int h = L >> 1;
@@ -47,9 +47,9 @@ __device__ void fft_dif(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
     const int lh = logL - 1;  // h = 2^lh
     for (int jj = t; jj < h * P; jj += NT) {
       const int p = jj >> lh, j = jj & (h - 1);
-      cplx<T> *Y = X + p * ldx;
-      cplx<T> w = cconj(ld<T>(tw, int64_t(j) * stride));
-      cplx<T> u = Y[pad(j)], v = Y[pad(j + h)];
+      cplx<float> *Y = X + p * ldx;
+      cplx<float> w = cconj(ld<float>(tw, int64_t(j) * stride));
+      cplx<float> u = Y[pad(j)], v = Y[pad(j + h)];
       Y[pad(j)] = cadd(u, v);
       Y[pad(j + h)] = cmul(csub(u, v), w);
     }
@@ -62,15 +62,15 @@ __device__ void fft_dif(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
     const int stride = maxL / (2 * h);
     for (int gg = t; gg < L4 * P; gg += NT) {
       const int p = gg >> lL4, g = gg & (L4 - 1);
-      cplx<T> *Y = X + p * ldx;
+      cplx<float> *Y = X + p * ldx;
       const int blk = g >> lq, pos = g & (q - 1);
       const int b0 = blk * 2 * h + pos;
-      cplx<T> w1 = cconj(ld<T>(tw, int64_t(pos) * stride));
-      cplx<T> w2 = cmul(w1, w1);
-      cplx<T> w3 = {w1.im, -w1.re};  // w1 * (-i)
-      cplx<T> a = Y[pad(b0)], b = Y[pad(b0 + q)], c = Y[pad(b0 + h)], d = Y[pad(b0 + h + q)];
-      cplx<T> a1 = cadd(a, c), c1 = cmul(csub(a, c), w1);
-      cplx<T> b1 = cadd(b, d), d1 = cmul(csub(b, d), w3);
+      cplx<float> w1 = cconj(ld<float>(tw, int64_t(pos) * stride));
+      cplx<float> w2 = cmul(w1, w1);
+      cplx<float> w3 = {w1.im, -w1.re};  // w1 * (-i)
+      cplx<float> a = Y[pad(b0)], b = Y[pad(b0 + q)], c = Y[pad(b0 + h)], d = Y[pad(b0 + h + q)];
+      cplx<float> a1 = cadd(a, c), c1 = cmul(csub(a, c), w1);
+      cplx<float> b1 = cadd(b, d), d1 = cmul(csub(b, d), w3);
       Y[pad(b0)] = cadd(a1, b1);
       Y[pad(b0 + q)] = cmul(csub(a1, b1), w2);
       Y[pad(b0 + h)] = cadd(c1, d1);
@@ -82,8 +82,8 @@ __device__ void fft_dif(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
 
 // In-place inverse FFT (e^{+2 pi i}, unscaled), bit-reversed in, natural out,
 // on P arrays X + p ldx.
-template <typename T, int NT, int P>
-__device__ void fft_dit(cplx<T> *X, int ldx, int L, const typename tab_t<T>::type *tw, int maxL) {
+template <int NT, int P>
+__device__ void fft_dit(cplx<float> *X, int ldx, int L, const float2 *tw, int maxL) {
   const int t = threadIdx.x;
   const int logL = ilog2(L);
   int h = 1;
@@ -91,8 +91,8 @@ __device__ void fft_dit(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
     const int L2 = L >> 1, lL2 = logL - 1;
     for (int jj = t; jj < L2 * P; jj += NT) {
       const int p = jj >> lL2, j = jj & (L2 - 1);
-      cplx<T> *Y = X + p * ldx;
-      cplx<T> u = Y[pad(2 * j)], v = Y[pad(2 * j + 1)];
+      cplx<float> *Y = X + p * ldx;
+      cplx<float> u = Y[pad(2 * j)], v = Y[pad(2 * j + 1)];
       Y[pad(2 * j)] = cadd(u, v);
       Y[pad(2 * j + 1)] = csub(u, v);
     }
@@ -105,17 +105,18 @@ __device__ void fft_dit(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
     const int lh = ilog2(h);
     for (int gg = t; gg < L4 * P; gg += NT) {
       const int p = gg >> lL4, g = gg & (L4 - 1);
-      cplx<T> *Y = X + p * ldx;
+      cplx<float> *Y = X + p * ldx;
       const int blk = g >> lh, pos = g & (h - 1);
       const int a0 = blk * 4 * h + pos;
-      cplx<T> w4 = ld<T>(tw, int64_t(pos) * stride);
-      cplx<T> w = cmul(w4, w4);
-      cplx<T> w4i = cmuli(w4);
-      cplx<T> a = Y[pad(a0)], b = Y[pad(a0 + h)], c = Y[pad(a0 + 2 * h)], d = Y[pad(a0 + 3 * h)];
-      cplx<T> tb = cmul(b, w), td = cmul(d, w);
-      cplx<T> a1 = cadd(a, tb), b1 = csub(a, tb);
-      cplx<T> c1 = cadd(c, td), d1 = csub(c, td);
-      cplx<T> tc = cmul(c1, w4), tdd = cmul(d1, w4i);
+      cplx<float> w4 = ld<float>(tw, int64_t(pos) * stride);
+      cplx<float> w = cmul(w4, w4);
+      cplx<float> w4i = cmuli(w4);
+      cplx<float> a = Y[pad(a0)], b = Y[pad(a0 + h)];
+      cplx<float> c = Y[pad(a0 + 2 * h)], d = Y[pad(a0 + 3 * h)];
+      cplx<float> tb = cmul(b, w), td = cmul(d, w);
+      cplx<float> a1 = cadd(a, tb), b1 = csub(a, tb);
+      cplx<float> c1 = cadd(c, td), d1 = csub(c, td);
+      cplx<float> tc = cmul(c1, w4), tdd = cmul(d1, w4i);
       Y[pad(a0)] = cadd(a1, tc);
       Y[pad(a0 + 2 * h)] = csub(a1, tc);
       Y[pad(a0 + h)] = cadd(b1, tdd);
@@ -128,10 +129,10 @@ __device__ void fft_dit(cplx<T> *X, int ldx, int L, const typename tab_t<T>::typ
 // Inverse length-r DFT of the values H[i][slot][p] (owned j1 = t + i NT) for
 // the P arrays p, in place in the registers; X holds P work arrays of stride
 // ldx in LDS.  conj_io conjugates input and output (the forward DFT).
-template <typename T, int NT, int MAXC, int P>
-__device__ void sub_idft(cplx<T> (&H)[MAXC][4][P], int slot, int r, cplx<T> *X, int ldx,
-                         int64_t boff, const typename tab_t<T>::type *blu,
-                         const typename tab_t<T>::type *tw, int maxL, bool conj_io) {
+template <int NT, int MAXC, int P>
+__device__ void sub_idft(cplx<float> (&H)[MAXC][4][P], int slot, int r, cplx<float> *X, int ldx,
+                         int64_t boff, const float2 *blu,
+                         const float2 *tw, int maxL, bool conj_io) {
   const int t = threadIdx.x;
   __syncthreads();  // X free
   if (boff < 0) {   // r is a power of two
@@ -143,36 +144,36 @@ __device__ void sub_idft(cplx<T> (&H)[MAXC][4][P], int slot, int r, cplx<T> *X, 
         const int pos = bits ? int(__brev(unsigned(j1)) >> (32 - bits)) : 0;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-          cplx<T> v = H[i][slot][p];
+          cplx<float> v = H[i][slot][p];
           X[p * ldx + pad(pos)] = conj_io ? cconj(v) : v;
         }
       }
     }
     __syncthreads();
-    fft_dit<T, NT, P>(X, ldx, r, tw, maxL);
+    fft_dit<NT, P>(X, ldx, r, tw, maxL);
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int j1 = t + i * NT;
       if (j1 < r) {
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-          cplx<T> v = X[p * ldx + pad(j1)];
+          cplx<float> v = X[p * ldx + pad(j1)];
           H[i][slot][p] = conj_io ? cconj(v) : v;
         }
       }
     }
   } else {
     const int L = blu_len(r);
-    const typename tab_t<T>::type *c = blu + boff;
-    const typename tab_t<T>::type *bh = c + r;
+    const float2 *c = blu + boff;
+    const float2 *bh = c + r;
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int j1 = t + i * NT;
       if (j1 < r) {
-        const cplx<T> cj = ld<T>(c, j1);
+        const cplx<float> cj = ld<float>(c, j1);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-          cplx<T> v = H[i][slot][p];
+          cplx<float> v = H[i][slot][p];
           if (conj_io) v = cconj(v);
           X[p * ldx + pad(j1)] = cmul(v, cj);
         }
@@ -180,25 +181,25 @@ __device__ void sub_idft(cplx<T> (&H)[MAXC][4][P], int slot, int r, cplx<T> *X, 
     }
     for (int jj = t; jj < (L - r) * P; jj += NT) {
       const int p = jj / (L - r), j = r + jj - p * (L - r);
-      X[p * ldx + pad(j)] = cplx<T>{T(0), T(0)};
+      X[p * ldx + pad(j)] = cplx<float>{0.0f, 0.0f};
     }
     __syncthreads();
-    fft_dif<T, NT, P>(X, ldx, L, tw, maxL);
+    fft_dif<NT, P>(X, ldx, L, tw, maxL);
     const int lL = ilog2(L);
     for (int jj = t; jj < L * P; jj += NT) {
       const int p = jj >> lL, j = jj & (L - 1);
-      X[p * ldx + pad(j)] = cmul(X[p * ldx + pad(j)], ld<T>(bh, j));
+      X[p * ldx + pad(j)] = cmul(X[p * ldx + pad(j)], ld<float>(bh, j));
     }
     __syncthreads();
-    fft_dit<T, NT, P>(X, ldx, L, tw, maxL);
+    fft_dit<NT, P>(X, ldx, L, tw, maxL);
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int j1 = t + i * NT;
       if (j1 < r) {
-        const cplx<T> cj = ld<T>(c, j1);
+        const cplx<float> cj = ld<float>(c, j1);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-          cplx<T> v = cmul(X[p * ldx + pad(j1)], cj);
+          cplx<float> v = cmul(X[p * ldx + pad(j1)], cj);
           H[i][slot][p] = conj_io ? cconj(v) : v;
         }
       }
@@ -238,18 +239,16 @@ __device__ __forceinline__ float expm1_map(float x) {
   }
   return r;
 }
-__device__ __forceinline__ float expm1_t(float x) { return expm1_map(x); }
 
-template <typename T>
-__device__ __forceinline__ T apply_epi(T x, int kind, T lam, T par) {
+__device__ __forceinline__ float apply_epi(float x, int kind, float lam, float par) {
   if (kind == GA_T_LOGNORMAL) {
-    T y = expm1_t(x - par * T(0.5));
-    return lam == T(1) ? y : lam * y;
+    float y = expm1_map(x - par * 0.5f);
+    return lam == 1.0f ? y : lam * y;
   }
   if (kind == GA_T_SQUARED_NORMAL) {
-    T d = x - par;
-    T y = d * d - T(1);
-    return lam == T(1) ? y : lam * y;
+    float d = x - par;
+    float y = d * d - 1.0f;
+    return lam == 1.0f ? y : lam * y;
   }
   return x;
 }
@@ -290,14 +289,14 @@ __device__ __forceinline__ bool decode_ring_block(int nrings, int npp, int &ring
 // direct terms summed before conjugate terms, each in increasing m.
 // fold_shells_own: one thread, one bin; the loads of four terms are issued
 // together at clamped addresses (one round when n > lmax).
-template <typename T, int NQ>
-__device__ __forceinline__ void fold_shells_own(const cplx<T> *__restrict__ Fu, int G, int nsh,
-                                                int k, int n, int lmax, cplx<T> (&g)[NQ]) {
+template <int NQ>
+__device__ __forceinline__ void fold_shells_own(const cplx<float> *__restrict__ Fu, int G, int nsh,
+                                                int k, int n, int lmax, cplx<float> (&g)[NQ]) {
   const int mc0 = k == 0 ? n : n - k;
   if (n > lmax) {
-    cplx<T> fd[NQ], fc[NQ];
-    const cplx<T> *a = Fu + int64_t(min(k, lmax)) * G;
-    const cplx<T> *c = Fu + int64_t(min(mc0, lmax)) * G;
+    cplx<float> fd[NQ], fc[NQ];
+    const cplx<float> *a = Fu + int64_t(min(k, lmax)) * G;
+    const cplx<float> *c = Fu + int64_t(min(mc0, lmax)) * G;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       fd[q] = a[min(q, nsh - 1)];
@@ -312,10 +311,10 @@ __device__ __forceinline__ void fold_shells_own(const cplx<T> *__restrict__ Fu, 
     return;
   }
   for (int m0 = k; m0 <= lmax; m0 += 4 * n) {
-    cplx<T> f[4][NQ];
+    cplx<float> f[4][NQ];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const cplx<T> *a = Fu + int64_t(min(m0 + u * n, lmax)) * G;
+      const cplx<float> *a = Fu + int64_t(min(m0 + u * n, lmax)) * G;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) f[u][q] = a[min(q, nsh - 1)];
     }
@@ -327,10 +326,10 @@ __device__ __forceinline__ void fold_shells_own(const cplx<T> *__restrict__ Fu, 
           if (q < nsh) g[q] = cadd(g[q], f[u][q]);
   }
   for (int m0 = mc0; m0 <= lmax; m0 += 4 * n) {
-    cplx<T> f[4][NQ];
+    cplx<float> f[4][NQ];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const cplx<T> *a = Fu + int64_t(min(m0 + u * n, lmax)) * G;
+      const cplx<float> *a = Fu + int64_t(min(m0 + u * n, lmax)) * G;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) f[u][q] = a[min(q, nsh - 1)];
     }
@@ -348,24 +347,24 @@ __device__ __forceinline__ void fold_shells_own(const cplx<T> *__restrict__ Fu, 
 // conjugate m = (j + 1) n - k); the partial sums meet in LDS and are added in
 // q order.  Result: bin k of shell q at X[q n + k].  X must hold 2 NT NQ
 // entries; every thread of the workgroup takes part.
-template <typename T, int NT, int NQ>
-__device__ __forceinline__ void fold_shells_coop(const cplx<T> *__restrict__ Fu, int G, int nsh,
-                                                 int n, int lmax, cplx<T> *X) {
+template <int NT, int NQ>
+__device__ __forceinline__ void fold_shells_coop(const cplx<float> *__restrict__ Fu, int G, int nsh,
+                                                 int n, int lmax, cplx<float> *X) {
   const int t = threadIdx.x;
   const int Q = NT / n, nitems = n * Q;  // nitems <= NT
   const int jmax = lmax / n;
-  cplx<T> d[NQ], c[NQ];
+  cplx<float> d[NQ], c[NQ];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) d[q] = c[q] = cplx<T>{T(0), T(0)};
+  for (int q = 0; q < NQ; ++q) d[q] = c[q] = cplx<float>{0.0f, 0.0f};
   if (t < nitems) {
     const int qq = t / n, k = t - qq * n;
     for (int j0 = qq; j0 <= jmax; j0 += 4 * Q) {
-      cplx<T> fd[4][NQ], fc[4][NQ];
+      cplx<float> fd[4][NQ], fc[4][NQ];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int j = j0 + u * Q;
-        const cplx<T> *a = Fu + int64_t(min(j * n + k, lmax)) * G;
-        const cplx<T> *b = Fu + int64_t(min((j + 1) * n - k, lmax)) * G;
+        const cplx<float> *a = Fu + int64_t(min(j * n + k, lmax)) * G;
+        const cplx<float> *b = Fu + int64_t(min((j + 1) * n - k, lmax)) * G;
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
           fd[u][q] = a[min(q, nsh - 1)];
@@ -392,11 +391,11 @@ __device__ __forceinline__ void fold_shells_coop(const cplx<T> *__restrict__ Fu,
     }
   }
   __syncthreads();
-  cplx<T> g[NQ];
+  cplx<float> g[NQ];
   if (t < n) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      cplx<T> sd = {T(0), T(0)}, sc = {T(0), T(0)};
+      cplx<float> sd = {0.0f, 0.0f}, sc = {0.0f, 0.0f};
       for (int j = 0; j < Q; ++j) sd = cadd(sd, X[(2 * q) * NT + j * n + t]);
       for (int j = 0; j < Q; ++j) sc = cadd(sc, X[(2 * q + 1) * NT + j * n + t]);
       g[q] = cadd(sd, sc);
@@ -409,15 +408,15 @@ __device__ __forceinline__ void fold_shells_coop(const cplx<T> *__restrict__ Fu,
   }
 }
 
-template <typename T, int NT, int MAXC, int P>
+template <int NT, int MAXC, int P>
 __global__ __launch_bounds__(NT) void ring_synth_kernel(
     int lmax, int nrings, const int64_t *__restrict__ ring_start,
     const int32_t *__restrict__ ring_n, const int64_t *__restrict__ blu_off,
-    const typename tab_t<T>::type *__restrict__ blu, const typename tab_t<T>::type *__restrict__ tw,
-    int maxL, int ldx, const cplx<T> *__restrict__ F, int S, int G, int nunit,
-    T *__restrict__ maps, int64_t npix, const ga_epilogue *__restrict__ epi) {
+    const float2 *__restrict__ blu, const float2 *__restrict__ tw,
+    int maxL, int ldx, const cplx<float> *__restrict__ F, int S, int G, int nunit,
+    float *__restrict__ maps, int64_t npix, const ga_epilogue *__restrict__ epi) {
   extern __shared__ char smem_raw[];
-  cplx<T> *X = reinterpret_cast<cplx<T> *>(smem_raw);
+  cplx<float> *X = reinterpret_cast<cplx<float> *>(smem_raw);
   int ring, unit;
   if (!decode_ring_block(nrings, nunit, ring, unit)) return;
   const int t = threadIdx.x;
@@ -427,46 +426,46 @@ __global__ __launch_bounds__(NT) void ring_synth_kernel(
   const int ngrp = (S + G - 1) / G;
   // pointer of shell sbase at m = 0; the unit's 2P shells are contiguous
   // because G is a multiple of 2P or G = S
-  const cplx<T> *Fu = F + (int64_t(ring) * ngrp + sbase / G) * (lmax + 1) * G + sbase % G;
+  const cplx<float> *Fu = F + (int64_t(ring) * ngrp + sbase / G) * (lmax + 1) * G + sbase % G;
   int nsh = S - sbase;
   if (nsh > 2 * P) nsh = 2 * P;
 
   // fold of the ring's coefficients into its n bins (see fold_shells_*):
   // small rings cooperatively through LDS, large rings per thread
   const bool coop = n <= NT / 2;
-  if (coop) fold_shells_coop<T, NT, 2 * P>(Fu, G, nsh, n, lmax, X);
+  if (coop) fold_shells_coop<NT, 2 * P>(Fu, G, nsh, n, lmax, X);
   __syncthreads();
-  cplx<T> H[MAXC][4][P];
+  cplx<float> H[MAXC][4][P];
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
     const int k1 = t + i * NT;
-    cplx<T> h[4][P];
+    cplx<float> h[4][P];
 #pragma unroll
     for (int k2 = 0; k2 < 4; ++k2) {
-      cplx<T> g[2 * P];
+      cplx<float> g[2 * P];
 #pragma unroll
-      for (int q = 0; q < 2 * P; ++q) g[q] = cplx<T>{T(0), T(0)};
+      for (int q = 0; q < 2 * P; ++q) g[q] = cplx<float>{0.0f, 0.0f};
       if (k1 < r) {
         const int k = k1 + r * k2;
         if (coop) {
 #pragma unroll
           for (int q = 0; q < 2 * P; ++q) g[q] = X[q * n + k];
         } else {
-          fold_shells_own<T, 2 * P>(Fu, G, nsh, k, n, lmax, g);
+          fold_shells_own<2 * P>(Fu, G, nsh, k, n, lmax, g);
         }
       }
 #pragma unroll
       for (int p = 0; p < P; ++p)
-        h[k2][p] = cplx<T>{g[2 * p].re - g[2 * p + 1].im, g[2 * p].im + g[2 * p + 1].re};
+        h[k2][p] = cplx<float>{g[2 * p].re - g[2 * p + 1].im, g[2 * p].im + g[2 * p + 1].re};
     }
     // radix-4 across k2 and twiddle w_n^{j2 k1} (k1 < r, so w2 = w1^2, w3 = w1^3)
-    const cplx<T> w1 = expi_q(k1 < r ? k1 : 0, n, T(0));
-    const cplx<T> w2 = cmul(w1, w1);
-    const cplx<T> w3 = cmul(w2, w1);
+    const cplx<float> w1 = expi_q(k1 < r ? k1 : 0, n, 0.0f);
+    const cplx<float> w2 = cmul(w1, w1);
+    const cplx<float> w3 = cmul(w2, w1);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      const cplx<T> s02 = cadd(h[0][p], h[2][p]), d02 = csub(h[0][p], h[2][p]);
-      const cplx<T> s13 = cadd(h[1][p], h[3][p]), d13 = cmuli(csub(h[1][p], h[3][p]));
+      const cplx<float> s02 = cadd(h[0][p], h[2][p]), d02 = csub(h[0][p], h[2][p]);
+      const cplx<float> s13 = cadd(h[1][p], h[3][p]), d13 = cmuli(csub(h[1][p], h[3][p]));
       H[i][0][p] = cadd(s02, s13);
       H[i][1][p] = cmul(cadd(d02, d13), w1);
       H[i][2][p] = cmul(csub(s02, s13), w2);
@@ -477,7 +476,7 @@ __global__ __launch_bounds__(NT) void ring_synth_kernel(
   // ---- four length-r inverse DFTs per pair
 #pragma unroll
   for (int j2 = 0; j2 < 4; ++j2)
-    sub_idft<T, NT, MAXC, P>(H, j2, r, X, ldx, boff, blu, tw, maxL, false);
+    sub_idft<NT, MAXC, P>(H, j2, r, X, ldx, boff, blu, tw, maxL, false);
 
   // ---- epilogue and store: pixel 4 j1 + j2 of each shell (epilogue
   // parameters are workgroup-uniform loads, read where they are used)
@@ -486,13 +485,21 @@ __global__ __launch_bounds__(NT) void ring_synth_kernel(
   for (int p = 0; p < P; ++p) {
     const int q0 = 2 * p, q1 = 2 * p + 1;
     int k0 = GA_T_NORMAL, kk1 = GA_T_NORMAL;
-    T l0 = T(1), a0 = T(0), l1 = T(1), a1 = T(0);
+    float l0 = 1.0f, a0 = 0.0f, l1 = 1.0f, a1 = 0.0f;
     if (epi) {
-      if (q0 < nsh) { k0 = epi[sbase + q0].kind; l0 = T(epi[sbase + q0].lamda); a0 = T(epi[sbase + q0].param); }
-      if (q1 < nsh) { kk1 = epi[sbase + q1].kind; l1 = T(epi[sbase + q1].lamda); a1 = T(epi[sbase + q1].param); }
+      if (q0 < nsh) {
+        k0 = epi[sbase + q0].kind;
+        l0 = float(epi[sbase + q0].lamda);
+        a0 = float(epi[sbase + q0].param);
+      }
+      if (q1 < nsh) {
+        kk1 = epi[sbase + q1].kind;
+        l1 = float(epi[sbase + q1].lamda);
+        a1 = float(epi[sbase + q1].param);
+      }
     }
-    T *out0 = maps + int64_t(sbase + q0) * npix + st;
-    T *out1 = maps + int64_t(sbase + q1) * npix + st;
+    float *out0 = maps + int64_t(sbase + q0) * npix + st;
+    float *out1 = maps + int64_t(sbase + q1) * npix + st;
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int j1 = t + i * NT;
@@ -500,8 +507,8 @@ __global__ __launch_bounds__(NT) void ring_synth_kernel(
 #pragma unroll
         for (int j2 = 0; j2 < 4; ++j2) {
           const int64_t pix = 4 * int64_t(j1) + j2;
-          if (q0 < nsh) out0[pix] = apply_epi<T>(H[i][j2][p].re, k0, l0, a0);
-          if (q1 < nsh) out1[pix] = apply_epi<T>(H[i][j2][p].im, kk1, l1, a1);
+          if (q0 < nsh) out0[pix] = apply_epi(H[i][j2][p].re, k0, l0, a0);
+          if (q1 < nsh) out1[pix] = apply_epi(H[i][j2][p].im, kk1, l1, a1);
         }
       }
     }
@@ -509,16 +516,16 @@ __global__ __launch_bounds__(NT) void ring_synth_kernel(
 }
 
 // Analysis: maps pair -> F[ring][m][s] = w e^{-i m phi0} DFT(f)_{m mod n}
-template <typename T, int NT, int MAXC>
+template <int NT, int MAXC>
 __global__ __launch_bounds__(NT) void ring_anal_kernel(
     int lmax, int nrings, const int64_t *__restrict__ ring_start,
     const int32_t *__restrict__ ring_n, const int32_t *__restrict__ ring_pnum,
     const int32_t *__restrict__ ring_pden, const int64_t *__restrict__ blu_off,
-    const typename tab_t<T>::type *__restrict__ blu, const typename tab_t<T>::type *__restrict__ tw,
-    int maxL, const T *__restrict__ maps, int S, int npp, int64_t npix, T weight,
-    cplx<T> *__restrict__ F) {
+    const float2 *__restrict__ blu, const float2 *__restrict__ tw,
+    int maxL, const float *__restrict__ maps, int S, int npp, int64_t npix, float weight,
+    cplx<float> *__restrict__ F) {
   extern __shared__ char smem_raw[];
-  cplx<T> *X = reinterpret_cast<cplx<T> *>(smem_raw);
+  cplx<float> *X = reinterpret_cast<cplx<float> *>(smem_raw);
   int ring, pair;
   if (!decode_ring_block(nrings, npp, ring, pair)) return;
   const int t = threadIdx.x;
@@ -528,20 +535,20 @@ __global__ __launch_bounds__(NT) void ring_anal_kernel(
   const int pnum = ring_pnum[ring], pden = ring_pden[ring];
   const int64_t boff = blu_off[r];
   const int64_t st = ring_start[ring];
-  const T *in0 = maps + int64_t(s0) * npix + st;
-  const T *in1 = maps + int64_t(s1) * npix + st;
+  const float *in0 = maps + int64_t(s0) * npix + st;
+  const float *in1 = maps + int64_t(s1) * npix + st;
 
   // x_{4 j1 + j2} = f0 + i f1; thread owns j1
-  cplx<T> H[MAXC][4][1];
+  cplx<float> H[MAXC][4][1];
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
     const int j1 = t + i * NT;
 #pragma unroll
     for (int j2 = 0; j2 < 4; ++j2) {
-      cplx<T> v = {T(0), T(0)};
+      cplx<float> v = {0.0f, 0.0f};
       if (j1 < r) {
         v.re = in0[4 * j1 + j2];
-        v.im = has1 ? in1[4 * j1 + j2] : T(0);
+        v.im = has1 ? in1[4 * j1 + j2] : 0.0f;
       }
       H[i][j2][0] = v;
     }
@@ -549,19 +556,19 @@ __global__ __launch_bounds__(NT) void ring_anal_kernel(
   // forward length-r DFTs of each decimated sequence
 #pragma unroll
   for (int j2 = 0; j2 < 4; ++j2)
-    sub_idft<T, NT, MAXC, 1>(H, j2, r, X, 0, boff, blu, tw, maxL, true);
+    sub_idft<NT, MAXC, 1>(H, j2, r, X, 0, boff, blu, tw, maxL, true);
   __syncthreads();
   // X_{k1 + r k2} = sum_{j2} (-i)^{j2 k2} e^{-2 pi i j2 k1 / n} D_{j2}[k1] -> LDS
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
     const int k1 = t + i * NT;
     if (k1 < r) {
-      const cplx<T> y0 = H[i][0][0];
-      const cplx<T> y1 = cmul(H[i][1][0], cconj(expi_q(k1, n, T(0))));
-      const cplx<T> y2 = cmul(H[i][2][0], cconj(expi_q((2 * k1) % n, n, T(0))));
-      const cplx<T> y3 = cmul(H[i][3][0], cconj(expi_q((3 * k1) % n, n, T(0))));
-      const cplx<T> s02 = cadd(y0, y2), d02 = csub(y0, y2);
-      const cplx<T> s13 = cadd(y1, y3), d13 = cmuli(csub(y3, y1));  // -i (y1 - y3)
+      const cplx<float> y0 = H[i][0][0];
+      const cplx<float> y1 = cmul(H[i][1][0], cconj(expi_q(k1, n, 0.0f)));
+      const cplx<float> y2 = cmul(H[i][2][0], cconj(expi_q((2 * k1) % n, n, 0.0f)));
+      const cplx<float> y3 = cmul(H[i][3][0], cconj(expi_q((3 * k1) % n, n, 0.0f)));
+      const cplx<float> s02 = cadd(y0, y2), d02 = csub(y0, y2);
+      const cplx<float> s13 = cadd(y1, y3), d13 = cmuli(csub(y3, y1));  // -i (y1 - y3)
       X[pad(k1)] = cadd(s02, s13);
       X[pad(k1 + r)] = cadd(d02, d13);
       X[pad(k1 + 2 * r)] = csub(s02, s13);
@@ -573,16 +580,16 @@ __global__ __launch_bounds__(NT) void ring_anal_kernel(
   for (int m = t; m <= lmax; m += NT) {
     const int k = m % n;
     const int kk = k ? n - k : 0;
-    const cplx<T> a = X[pad(k)], b = cconj(X[pad(kk)]);
-    cplx<T> d0 = {T(0.5) * (a.re + b.re), T(0.5) * (a.im + b.im)};
-    cplx<T> d1 = {T(0.5) * (a.im - b.im), T(-0.5) * (a.re - b.re)};  // (a - b) / (2i)
-    const cplx<T> ph = pnum ? cconj(expi_q(m % pden, pden, T(0))) : cplx<T>{T(1), T(0)};
-    cplx<T> *f = F + (int64_t(ring) * (lmax + 1) + m) * S;
-    cplx<T> v0 = cmul(d0, ph);
-    f[s0] = cplx<T>{weight * v0.re, weight * v0.im};
+    const cplx<float> a = X[pad(k)], b = cconj(X[pad(kk)]);
+    cplx<float> d0 = {0.5f * (a.re + b.re), 0.5f * (a.im + b.im)};
+    cplx<float> d1 = {0.5f * (a.im - b.im), -0.5f * (a.re - b.re)};  // (a - b) / (2i)
+    const cplx<float> ph = pnum ? cconj(expi_q(m % pden, pden, 0.0f)) : cplx<float>{1.0f, 0.0f};
+    cplx<float> *f = F + (int64_t(ring) * (lmax + 1) + m) * S;
+    cplx<float> v0 = cmul(d0, ph);
+    f[s0] = cplx<float>{weight * v0.re, weight * v0.im};
     if (has1) {
-      cplx<T> v1 = cmul(d1, ph);
-      f[s1] = cplx<T>{weight * v1.re, weight * v1.im};
+      cplx<float> v1 = cmul(d1, ph);
+      f[s1] = cplx<float>{weight * v1.re, weight * v1.im};
     }
   }
 }
@@ -871,11 +878,11 @@ __global__ __launch_bounds__(NT) void ring_synth2_kernel(
       y[q] = X[q * ldx + pad(j1)];
       if (BLU) y[q] = cmul(y[q], cj);
     }
-    out0[j1] = resid4(ref, int64_t(sbase) * npix + st, j1, float4{apply_epi<float>(y[0].re, k0, l0, a0), apply_epi<float>(y[1].re, k0, l0, a0),
-                      apply_epi<float>(y[2].re, k0, l0, a0), apply_epi<float>(y[3].re, k0, l0, a0)});
+    out0[j1] = resid4(ref, int64_t(sbase) * npix + st, j1, float4{apply_epi(y[0].re, k0, l0, a0), apply_epi(y[1].re, k0, l0, a0),
+                      apply_epi(y[2].re, k0, l0, a0), apply_epi(y[3].re, k0, l0, a0)});
     if (two)
-      out1[j1] = resid4(ref, int64_t(sbase + 1) * npix + st, j1, float4{apply_epi<float>(y[0].im, kk1, l1, a1), apply_epi<float>(y[1].im, kk1, l1, a1),
-                        apply_epi<float>(y[2].im, kk1, l1, a1), apply_epi<float>(y[3].im, kk1, l1, a1)});
+      out1[j1] = resid4(ref, int64_t(sbase + 1) * npix + st, j1, float4{apply_epi(y[0].im, kk1, l1, a1), apply_epi(y[1].im, kk1, l1, a1),
+                        apply_epi(y[2].im, kk1, l1, a1), apply_epi(y[3].im, kk1, l1, a1)});
   }
 }
 
@@ -1170,11 +1177,11 @@ __global__ __launch_bounds__(NT, 4) void ring_synth_wide_kernel(
   for (int i = 0; i < C; ++i) {
     const int j1 = t + i * NT;
     const cplx<float> y[4] = {res[i][0], res[i][1], X[pad(j1)], X[ldx + pad(j1)]};
-    out0[j1] = resid4(ref, int64_t(sbase) * npix + st, j1, float4{apply_epi<float>(y[0].re, k0, l0, a0), apply_epi<float>(y[1].re, k0, l0, a0),
-                      apply_epi<float>(y[2].re, k0, l0, a0), apply_epi<float>(y[3].re, k0, l0, a0)});
+    out0[j1] = resid4(ref, int64_t(sbase) * npix + st, j1, float4{apply_epi(y[0].re, k0, l0, a0), apply_epi(y[1].re, k0, l0, a0),
+                      apply_epi(y[2].re, k0, l0, a0), apply_epi(y[3].re, k0, l0, a0)});
     if (two)
-      out1[j1] = resid4(ref, int64_t(sbase + 1) * npix + st, j1, float4{apply_epi<float>(y[0].im, kk1, l1, a1), apply_epi<float>(y[1].im, kk1, l1, a1),
-                        apply_epi<float>(y[2].im, kk1, l1, a1), apply_epi<float>(y[3].im, kk1, l1, a1)});
+      out1[j1] = resid4(ref, int64_t(sbase + 1) * npix + st, j1, float4{apply_epi(y[0].im, kk1, l1, a1), apply_epi(y[1].im, kk1, l1, a1),
+                        apply_epi(y[2].im, kk1, l1, a1), apply_epi(y[3].im, kk1, l1, a1)});
   }
 }
 
@@ -1388,11 +1395,11 @@ __global__ __launch_bounds__(NT, (NT == 256 && C == 4) ? 3 : 4) void ring_synth_
       cplx<float> v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = cmul(y[c][q], cj);
-      out0[j1] = resid4(ref, int64_t(sbase) * npix + st, j1, float4{apply_epi<float>(v[0].re, k0, l0, a0), apply_epi<float>(v[1].re, k0, l0, a0),
-                        apply_epi<float>(v[2].re, k0, l0, a0), apply_epi<float>(v[3].re, k0, l0, a0)});
+      out0[j1] = resid4(ref, int64_t(sbase) * npix + st, j1, float4{apply_epi(v[0].re, k0, l0, a0), apply_epi(v[1].re, k0, l0, a0),
+                        apply_epi(v[2].re, k0, l0, a0), apply_epi(v[3].re, k0, l0, a0)});
       if (two)
-        out1[j1] = resid4(ref, int64_t(sbase + 1) * npix + st, j1, float4{apply_epi<float>(v[0].im, kk1, l1, a1), apply_epi<float>(v[1].im, kk1, l1, a1),
-                          apply_epi<float>(v[2].im, kk1, l1, a1), apply_epi<float>(v[3].im, kk1, l1, a1)});
+        out1[j1] = resid4(ref, int64_t(sbase + 1) * npix + st, j1, float4{apply_epi(v[0].im, kk1, l1, a1), apply_epi(v[1].im, kk1, l1, a1),
+                          apply_epi(v[2].im, kk1, l1, a1), apply_epi(v[3].im, kk1, l1, a1)});
     }
   }
 }
@@ -1777,28 +1784,26 @@ int launch_ring_synth2_f32(const ga_plan *p, int S, int G, const float *F, float
   return rc;
 }
 
-template <typename T>
-int launch_ring(const ga_plan *p, int S, int G, const void *in, void *out, const ga_epilogue *epi,
-                bool anal, hipStream_t stream) {
-  static_assert(sizeof(T) == 4, "the FP64 ring stages are in ringfft64.hip");
+int launch_ring(const ga_plan *p, int S, int G, const float *in, float *out,
+                const ga_epilogue *epi, bool anal, hipStream_t stream) {
   const float2 *blu = p->d_blu32, *tw = p->d_tw32;
   const int max_r = p->max_r;
   if (anal) {
     const int npp = (S + 1) / 2;
     const int nblk = 8 * ((p->nrings + 7) / 8) * npp;
     // analysis assembles the full ring (n = 4 r <= 4 nside) in LDS as well
-    const size_t lds = size_t(padded_len(std::max(p->max_L, 4 * p->nside))) * 2 * sizeof(T);
+    const size_t lds = size_t(padded_len(std::max(p->max_L, 4 * p->nside))) * 2 * sizeof(float);
     GA_REQUIRE(lds <= 160 * 1024, GA_ERR_UNSUPPORTED,
                "ring analysis needs %zu bytes of LDS (nside %d)", lds, p->nside);
-#define GA_ANAL_LAUNCH(NT_, MAXC_)                                                             \
-  do {                                                                                        \
-    auto kfn = ring_anal_kernel<T, NT_, MAXC_>;                                               \
-    GA_CHECK_HIP(hipFuncSetAttribute((const void *)kfn,                                       \
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));  \
-    hipLaunchKernelGGL(kfn, dim3(nblk), dim3(NT_), lds, stream, p->lmax, p->nrings,           \
-                       p->d_ring_start, p->d_ring_n, p->d_ring_pnum, p->d_ring_pden,          \
-                       p->d_blu_off, blu, tw, p->tw_len, (const T *)in, S, npp, p->npix,       \
-                       T(4.0 * M_PI / double(p->npix)), (cplx<T> *)out);                       \
+#define GA_ANAL_LAUNCH(NT_, MAXC_)                                                         \
+  do {                                                                                     \
+    auto kfn = ring_anal_kernel<NT_, MAXC_>;                                               \
+    GA_CHECK_HIP(hipFuncSetAttribute((const void *)kfn,                                    \
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));\
+    hipLaunchKernelGGL(kfn, dim3(nblk), dim3(NT_), lds, stream, p->lmax, p->nrings,        \
+                       p->d_ring_start, p->d_ring_n, p->d_ring_pnum, p->d_ring_pden,       \
+                       p->d_blu_off, blu, tw, p->tw_len, in, S, npp, p->npix,              \
+                       float(4.0 * M_PI / double(p->npix)), (cplx<float> *)out);           \
   } while (0)
     if (max_r <= 256) GA_ANAL_LAUNCH(256, 1);
     else if (max_r <= 1024) GA_ANAL_LAUNCH(256, 4);
@@ -1813,34 +1818,30 @@ int launch_ring(const ga_plan *p, int S, int G, const void *in, void *out, const
   // P work arrays fit in LDS
   const int ldx = padded_len(p->max_L);
   int P = 1;
-  // FP32 with shells grouped by 4 or more: 2 pairs per workgroup up to
+  // shells grouped by 4 or more: 2 pairs per workgroup up to
   // r = 2048 (register budget), else 1
-  if (sizeof(T) == 4 && G % 4 == 0 && S > 2 && max_r <= 2048 &&
-      size_t(2) * ldx * 2 * sizeof(T) <= 128 * 1024)
+  if (G % 4 == 0 && S > 2 && max_r <= 2048 && size_t(2) * ldx * 2 * sizeof(float) <= 128 * 1024)
     P = 2;
   GA_REQUIRE(G == S || G % (2 * P) == 0, GA_ERR_INVALID, "shell group %d incompatible", G);
   const int nunit = (S + 2 * P - 1) / (2 * P);
   const int nblk = 8 * ((p->nrings + 7) / 8) * nunit;
   // P work arrays; the cooperative fold of small rings needs 4 P NT entries
-  const size_t lds0 = size_t(P) * ldx * 2 * sizeof(T);
+  const size_t lds0 = size_t(P) * ldx * 2 * sizeof(float);
   GA_REQUIRE(lds0 <= 160 * 1024, GA_ERR_UNSUPPORTED, "ring synthesis needs %zu bytes of LDS", lds0);
-#define GA_SYNTH_LAUNCH(NT_, MAXC_, P_)                                                        \
-  do {                                                                                        \
-    auto kfn = ring_synth_kernel<T, NT_, MAXC_, P_>;                                          \
-    const size_t lds = std::max(lds0, size_t(4) * P_ * NT_ * 2 * sizeof(T));                  \
-    GA_CHECK_HIP(hipFuncSetAttribute((const void *)kfn,                                       \
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));  \
-    hipLaunchKernelGGL(kfn, dim3(nblk), dim3(NT_), lds, stream, p->lmax, p->nrings,           \
-                       p->d_ring_start, p->d_ring_n, p->d_blu_off, blu, tw, p->tw_len, ldx,    \
-                       (const cplx<T> *)in, S, G, nunit, (T *)out, p->npix, epi);             \
+#define GA_SYNTH_LAUNCH(NT_, MAXC_, P_)                                                    \
+  do {                                                                                     \
+    auto kfn = ring_synth_kernel<NT_, MAXC_, P_>;                                          \
+    const size_t lds = std::max(lds0, size_t(4) * P_ * NT_ * 2 * sizeof(float));           \
+    GA_CHECK_HIP(hipFuncSetAttribute((const void *)kfn,                                    \
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));\
+    hipLaunchKernelGGL(kfn, dim3(nblk), dim3(NT_), lds, stream, p->lmax, p->nrings,        \
+                       p->d_ring_start, p->d_ring_n, p->d_blu_off, blu, tw, p->tw_len, ldx,\
+                       (const cplx<float> *)in, S, G, nunit, out, p->npix, epi);           \
   } while (0)
-  if constexpr (sizeof(T) == 4) {
-    if (P == 2) {
-      if (max_r <= 512) GA_SYNTH_LAUNCH(256, 2, 2);
-      else GA_SYNTH_LAUNCH(512, 4, 2);
-    }
-  }
-  if (P == 1) {
+  if (P == 2) {
+    if (max_r <= 512) GA_SYNTH_LAUNCH(256, 2, 2);
+    else GA_SYNTH_LAUNCH(512, 4, 2);
+  } else {
     if (max_r <= 256) GA_SYNTH_LAUNCH(256, 1, 1);
     else if (max_r <= 1024) GA_SYNTH_LAUNCH(256, 4, 1);
     else if (max_r <= 2048) GA_SYNTH_LAUNCH(256, 8, 1);
@@ -1862,7 +1863,7 @@ int launch_ring_synth_f32(const ga_plan *p, int S, int G, const float *F, float 
     if (rc != GA_ERR_UNSUPPORTED) return rc;
     clear_error();
   }
-  return launch_ring<float>(p, S, G, F, maps, epi, false, s);
+  return launch_ring(p, S, G, F, maps, epi, false, s);
 }
 // out = ref - synthesis(F) in one pass (the residual of the analysis
 // iterations); GA_ERR_UNSUPPORTED (nothing launched) when the fused-pass form
@@ -1883,7 +1884,7 @@ int launch_ring_anal_f32(const ga_plan *p, int S, const float *maps, const doubl
     clear_error();
   }
   if (pixw) return GA_ERR_UNSUPPORTED;  // the first form does not weight
-  return launch_ring<float>(p, S, S, maps, F, nullptr, true, s);
+  return launch_ring(p, S, S, maps, F, nullptr, true, s);
 }
 
 }  // namespace ga
