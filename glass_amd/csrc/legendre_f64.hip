@@ -32,7 +32,7 @@ namespace ga {
 namespace {
 
 constexpr int kRows = 8;           // rows per batch of scalar loads
-constexpr int64_t kManyWaves = 16384;  // see launch_legendre_synth_f64
+constexpr int64_t kManyWaves = 12288;  // see launch_legendre_synth_f64
 
 enum { kPlain, kNorm, kDiff };  // forms of the recurrence
 
@@ -181,10 +181,10 @@ int launch_legendre_synth_f64(const ga_plan *p, const double *alm, double *F, do
                               size_t scratch_doubles, hipStream_t stream) {
   // The normalised form saves an operation in five and, with two pairs per
   // lane, half the scalar loads, but costs the launch of the scaling pass and
-  // the wait between the two, and half the waves.  Measured (whole alm2map):
-  // nside 256, lmax 512 (4104 waves of one pair per lane): plain 34 us,
-  // normalised 69; nside 512, lmax 1023 (16384 waves): 142 and 133 us; nside
-  // 1024, lmax 2048: 991 and 763 us.
+  // the wait between the two, and half the waves.  Whole alm2map by waves of one
+  // pair per lane, plain / normalised: 4104 (nside 256, lmax 512) 35 / 59 us; 9000
+  // (300, 899) 100 / 109; 10413 (400, 800) 112 / 110; 12816 (512, 800) 114 / 113; 14416
+  // (512, 900) 145 / 126; 16384 (512, 1023) 158 / 147; 35232 (1024, 1100) 373 / 316.
   const int64_t waves = int64_t(p->lmax + 1) * ((p->npairs + 63) / 64);
   if (waves < kManyWaves || scratch_doubles < size_t(2 * p->nalm))
     return launch<1, false>(p, alm, F, stream);
