@@ -143,8 +143,9 @@ __global__ __launch_bounds__(64 * kAWaves, 1) void legendre_anal_f16_kernel(
   // LDS: per wave the transposed slab lam[parity][l' (32)][pair (64)], each
   // value as its two FP16 halves in one word (a 16-bit store costs the LDS as
   // much as a 32-bit one: the two halves in arrays of their own took twice the
-  // stores; 7.85 -> 7.55 ms per analysis of 64 maps at nside 1024, lmax 2047), rows padded by 4 words so that the 16-byte A reads of 16
-  // consecutive lanes (rows 272 bytes apart) fall in distinct banks (17 KB);
+  // stores; 7.85 -> 7.55 ms per analysis of 64 maps at nside 1024, lmax 2047),
+  // rows padded by 4 words so that the 16-byte A reads of 16 consecutive lanes
+  // (rows 272 bytes apart) fall in distinct banks (17 KB);
   // after the MFMAs of a slab the same memory holds the waves' D tiles for
   // the fixed-order sum.  Recurrence coefficients gam_l are the same for
   // every wave of the workgroup (one m): one double buffer of one slab,

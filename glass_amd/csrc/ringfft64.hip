@@ -416,7 +416,12 @@ static int launch_anal64(const ga_plan *p, const double *maps, const double *pix
   return GA_OK;
 }
 
-// threads and k1 values per thread by the longest ring
+// Threads and k1 values per thread by the longest ring.  Whole alm2map at a small
+// band limit (the rings are most of it), against half as many threads with twice
+// the values and twice as many with half of them: nside 128 15.2, 15.2, 14.9 us; 200
+// 21.6, 24.5, 26.0; 300 33.6, 40.9, 40.5; 512 43.8, 50.8, 52.8; 1024 124, 142, 159; 2048
+// 681, 776, 963; the analysis likewise (below 129 64 threads are as good for the
+// synthesis, but 17.1 against 15.6 us for the analysis).
 #define GA_RING64_SIZES(FN, ...)                                                   \
   do {                                                                            \
     if (p->max_r <= 64) return FN<64, 1>(__VA_ARGS__);                            \
