@@ -3,8 +3,8 @@
 // p the parity of l - m, F the weighted, phase-removed ring coefficients.
 //
 // A workgroup of up to four waves takes one m; a lane owns RPL ring pairs, whose
-// recurrences (the normalised form y_l = lambda_l / c_l, two operations a step)
-// and Q stay in registers.  The sum runs over lanes, so each lane first adds
+// recurrences (the normalised form y_l = lambda_l / c_l, two operations a step,
+// norm_step) and Q stay in registers.  The sum runs over lanes, so each lane first adds
 // its own pairs for kRows rows of l (32 real sums in registers), and the wave
 // then reduces all 32 sums at once: every exchange halves the number of sums
 // a lane carries while it adds the partner's half (permlane swaps, then DPP
@@ -136,8 +136,8 @@ int launch_legendre_anal_f64(const ga_plan *p, const double *F, double *alm, dou
                              bool accumulate, hipStream_t stream) {
   // the fewest pairs per lane whose four waves cover an m: fewer need several
   // workgroups and partial sums per m, twice as many halve the waves (whole
-  // map2alm at nside 256, lmax 512: 57 us, 65 with twice as many; nside 512,
-  // lmax 1023: 167 and 204 us)
+  // map2alm, and with twice as many: nside 128, lmax 256 27 and 28 us; 256, 512 54
+  // and 65; 300, 767 114 and 150; 512, 1023 180 and 220)
   int rpl = 1;
   while (rpl < 8 && 256 * rpl < p->npairs) rpl *= 2;
   const int nw = std::min(4, (p->npairs + 64 * rpl - 1) / (64 * rpl));

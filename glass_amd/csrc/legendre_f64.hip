@@ -14,7 +14,7 @@
 // instead of three, against alm that a first pass has multiplied by c_l; the
 // plain form a (x lambda_{l-1} - b lambda_{l-2}) reads the alm as they are and
 // saves that launch.  (As (a x) lambda_{l-1} - (a b) lambda_{l-2} it would be one
-// operation deep instead of two, but with an error larger by 4 to 25 %.)
+// operation deep instead of two, but the sums' errors 3 to 17 % larger.)
 //
 // Bound: FP64 issue, 4 (NORM) or 5 operations per (l, m, ring pair).  Measured at
 // nside 1024, lmax 2048: 705 us (one pair per lane, a test of the scale and

@@ -1469,8 +1469,9 @@ int launch_blu_class(const ga_plan *p, const int32_t *list, int nlist, int max_r
 //
 // Bound: the unfolding as much as the transforms.  64 maps at nside 1024, lmax
 // 2047: power-of-two rings 2.28 ms, Bluestein rings 2.49 ms (2.39 and 2.65 with
-// 64-bit remainders and divisions in the ring phases); without the unfolding
-// 1.02 and 1.86, without the transforms 2.31 and 1.59.
+// 64-bit remainders and divisions in the ring phases).  Parts, measured beside
+// 2.36 and 2.52 ms for the whole: without the unfolding 1.02 and 1.86, without the
+// transforms 2.31 and 1.59.
 template <int NT, int C, bool BLU>
 __global__ __launch_bounds__(NT, (NT == 256 && C >= 4) ? 3 : 4) void ring_anal2_kernel(
     int lmax, const int32_t *__restrict__ ring_list, int nlist,
